@@ -739,16 +739,500 @@ __global__ __launch_bounds__(kPrefillThreads, D > 128 ? 1 : (D > 64 && QF32 ? 2 
     }
 }
 
-template <int D, int KV>
-void launch(const PrefillArgs& a, bool qf32, dim3 grid, hipStream_t s) {
-    if (qf32) chunked_prefill_kernel<D, KV, true><<<grid, kPrefillThreads, 0, s>>>(a);
-    else chunked_prefill_kernel<D, KV, false><<<grid, kPrefillThreads, 0, s>>>(a);
+// ---- calls with few workgroups: every wave streams keys of its own ------------------------------
+//
+// The kernel above gives a workgroup's waves one stream of keys and different units; a call whose
+// workgroups do not fill the chip (one 512-token chunk of a Llama-shaped layer is 128 of them) then
+// waits on the serial chain over the keys, about 0.92 us per pair of blocks for a workgroup alone
+// on its CU. Here a workgroup takes NU = 4 units (2 for head_dim 256) and its 8 waves split the
+// keys: wave w streams pairs w, w + 8, .. of the block list through an LDS slot of its own and
+// computes all four units on them, and the waves' (max, sum, O) are added up through LDS at the
+// end. No wave waits for another in the stream (eight waves stepping together behind a barrier
+// measured 59 us where this one takes 46), a K operand read from LDS feeds four units and a V
+// operand is converted to fp16 once for four. One slot a wave is enough: the next pair's K loads
+// go out when the QK products have read the slot's K, its V loads after the PV products, and the
+// SIMD's other wave runs while they land.
+//
+// What bounds it: VALU issue (softmax, V conversion) and MFMA, which two waves a SIMD overlap only
+// in part: about 2300 clocks per pair and wave against 1400 of VALU and 1020 of MFMA. A 512-token
+// chunk on 3333 tokens, Llama shape (32 / 8 heads of 128, bf16): 109.5 -> 46 us (660 TFLOP/s); 20
+// tokens on 8000: 220 -> 71; int8 cache, 512 on 2000: 109 -> 44.
+
+// LDS-direct loads of one tile of SEG KiB, 16 bytes a lane: segment j at immediate offset 1024 j,
+// which advances both the memory and the LDS address; off0 / off1 are the lane's offset within an
+// even / odd segment (the layouts repeat from there on).
+template <int SEG>
+__device__ __forceinline__ void lds_load_tile(u32x4_t r, uint32_t off0, uint32_t off1, uint32_t m0) {
+    uint32_t saved;
+    if constexpr (SEG == 1) {
+        asm volatile(
+            "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+            "buffer_load_dwordx4 %3, %1, 0 offen lds\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(saved)
+            : "s"(r), "s"(m0), "v"(off0)
+            : "memory");
+    } else if constexpr (SEG == 2) {
+        asm volatile(
+            "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+            "buffer_load_dwordx4 %3, %1, 0 offen lds\n\t"
+            "buffer_load_dwordx4 %4, %1, 0 offen offset:1024 lds\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(saved)
+            : "s"(r), "s"(m0), "v"(off0), "v"(off1)
+            : "memory");
+    } else if constexpr (SEG == 4) {
+        asm volatile(
+            "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+            "buffer_load_dwordx4 %3, %1, 0 offen lds\n\t"
+            "buffer_load_dwordx4 %4, %1, 0 offen offset:1024 lds\n\t"
+            "buffer_load_dwordx4 %3, %1, 0 offen offset:2048 lds\n\t"
+            "buffer_load_dwordx4 %4, %1, 0 offen offset:3072 lds\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(saved)
+            : "s"(r), "s"(m0), "v"(off0), "v"(off1)
+            : "memory");
+    } else {
+        static_assert(SEG == 8, "tiles of 1, 2, 4 or 8 KiB");
+        lds_load_tile<4>(r, off0, off1, m0);
+        lds_load_tile<4>(r, off0 + 4096, off1 + 4096, m0 + 4096);
+    }
+}
+
+// Units of a workgroup (each wave holds the accumulators of all of them) and its waves: two a SIMD,
+// one where 512 registers are needed (head_dim 256, or the low parts of fp32 queries).
+__host__ __device__ constexpr int wave_units(int d) { return d > 128 ? 2 : 4; }
+template <int D, bool QF32> __host__ __device__ constexpr int wave_waves() { return D > 128 || (D > 64 && QF32) ? 4 : 8; }
+
+// LDS of the kernel, one dynamic array: the compiler, which would see that only one workgroup fits
+// a CU, otherwise allots 512 registers a wave and moves the accumulators between the two halves of
+// the register file on every step.
+template <int D, int KV, bool QF32> struct WaveLds {
+    using TL = PrefillTile<D, MfmaRaw<KV>::kElt>;
+    static constexpr int WAVES = wave_waves<D, QF32>();
+    static constexpr int UNITS = wave_units(D);
+    static constexpr int NST = D / 16;                           // 16-byte words per lane of a unit's state
+    static constexpr int STATES = (WAVES > 4 ? 4 : 3) * UNITS;   // states exchanged at a time
+    static constexpr int TILES = WAVES * TL::SLOT > STATES * NST * 64 ? WAVES * TL::SLOT : STATES * NST * 64;
+    static constexpr int Q = UNITS * (D / 32) * 64;
+    static constexpr int KCH = KV == PA_DTYPE_INT8 ? 512 : 1024;  // block ids (and int8 scales) at a time
+    static constexpr int PAD = 4 * WAVES;                        // blocks a wave's last steps may reach past them
+    uint4 tile[TILES];  // a pair of blocks per wave (PrefillTile slot), then the states
+    union {
+        uint4 q[Q];              // Q operands
+        float2 ml[STATES * 64];  // the states' (max, row sum)
+    };
+    int ids[KCH + PAD];
+    float ksc[KV == PA_DTYPE_INT8 ? KCH + PAD : 1], vlg[KV == PA_DTYPE_INT8 ? KCH + PAD : 1],
+        vrc[KV == PA_DTYPE_INT8 ? KCH + PAD : 1];
+};
+
+template <int D, int KV, bool QF32>
+__global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>() / 4)) void chunked_prefill_wave_kernel(const PrefillArgs a) {
+    using Raw = MfmaRaw<KV>;
+    constexpr int ELT = Raw::kElt;
+    constexpr int NSLAB = D / 32;
+    constexpr int NT = D / 16;
+    constexpr int TILE = 16 * D;
+    constexpr int NU = wave_units(D);
+    using KR = typename Raw::K;
+    using TL = PrefillTile<D, ELT>;
+    constexpr int SEG = TL::SPT;             // KiB of a tile
+    using L = WaveLds<D, KV, QF32>;
+    constexpr int WAVES = L::WAVES, NST = L::NST, KCH = L::KCH, kPad = L::PAD;
+    extern __shared__ __align__(16) char wave_lds[];
+    L& sh = *reinterpret_cast<L*>(wave_lds);
+    uint4* const s_tile = sh.tile;
+    uint4* const s_q = sh.q;
+    float2* const s_ml = sh.ml;
+    int* const s_ids = sh.ids;
+    float *const s_ksc = sh.ksc, *const s_vlg = sh.vlg, *const s_vrc = sh.vrc;
+
+    // Workgroup -> (sequence, KV head) group gi and unit group qg, the ones with the most keys first:
+    // as above every group runs on XCD gi mod 8, where its workgroups share its K/V in one L2, but for
+    // the last num_groups mod 8 groups, whose workgroups are dealt to the XCDs in equal runs.
+    const int qgs = a.num_qgroups, xcd = blockIdx.x & 7, whole = a.num_groups >> 3;
+    int wk = blockIdx.x >> 3, gi;
+    if (wk < whole * qgs) {
+        gi = xcd + 8 * (wk / qgs);
+        wk %= qgs;
+    } else {
+        const int rest = (a.num_groups & 7) * qgs, per = (rest + 7) >> 3;
+        const int j = xcd * per + wk - whole * qgs;
+        if (j >= rest) return;
+        gi = 8 * whole + j / qgs;
+        wk = j % qgs;
+    }
+    const int qg = qgs - 1 - wk;
+    const int seq = gi / a.num_kv_heads, kvh = gi - seq * a.num_kv_heads;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q4 = lane >> 4, n = lane & 15;
+    const int G = a.group, Hkv = a.num_kv_heads, Hq = Hkv * G;
+
+    const int q0 = a.q_start_loc[seq];
+    const int Lc = a.q_start_loc[seq + 1] - q0;
+    const int P = max(a.prefix_lens[seq], 0);
+    const int T = min(P + Lc, a.max_blocks_per_seq * 16);
+    const bool causal = a.mask_mode == 0 || (a.mask_mode == 1 && P > 0);
+    const float c2 = a.scale * 1.4426950408889634f;
+    // Unit k: query head kvh G + u % G of query tile u / G, u = 4 qg + k. One past the chunk's tiles has
+    // no valid query: computed like the others, never stored.
+    int head[NU], i0[NU], nq[NU];
+#pragma unroll
+    for (int k = 0; k < NU; k++) {
+        const int u = NU * qg + k, qt = u / G;
+        head[k] = kvh * G + (u - qt * G);
+        i0[k] = 16 * qt;
+        nq[k] = max(0, min(16, Lc - i0[k]));
+    }
+    if (i0[0] >= Lc) return;
+    const int iew = min(Lc, i0[NU - 1] + 16);
+    const int kmax = causal ? min(T, P + iew) : T;
+    const int nkb = (kmax + 15) / 16;
+    const int klim_lo = causal ? min(T, P + i0[0] + 1) : T;
+    const int krow0 = (n & 3) + 8 * (n >> 3), kblk = (n >> 2) & 1;
+    const int pblk = q4 & 1, ptok = 8 * (q4 >> 1);
+    const int32_t* table = a.block_tables + static_cast<int64_t>(seq) * a.max_blocks_per_seq;
+    const char* kc = static_cast<const char*>(a.k_cache);
+    const char* vc = static_cast<const char*>(a.v_cache);
+
+    // Q operands: wave w stages unit w's in LDS, in the order the lanes read them (held in registers
+    // they would push the accumulators out of the 256 that VALU and MFMA both address); the low
+    // parts of fp32 queries stay in registers.
+    bf16x8_t qlo[NU][QF32 ? NSLAB : 1];
+#pragma unroll
+    for (int k = 0; k < NU; k++) {
+        if (!QF32 && k != wave) continue;
+        const bool qvalid = n < nq[k];
+        const int64_t qrow = (static_cast<int64_t>(q0 + (qvalid ? i0[k] + n : 0)) * Hq + head[k]) * D;
+#pragma unroll
+        for (int sl = 0; sl < NSLAB; sl++) {
+            const int d0 = 32 * sl + 8 * q4;
+            uint4 hi;
+            if constexpr (QF32) {
+                const float4* qp = reinterpret_cast<const float4*>(static_cast<const float*>(a.q) + qrow + d0);
+                const float4 w0 = qp[0], w1 = qp[1];
+                const float x[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+                uint32_t hh[4], ll[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    hh[e] = pack_bf16_trunc(x[2 * e], x[2 * e + 1]);
+                    const float r0 = x[2 * e] - __uint_as_float(__float_as_uint(x[2 * e]) & 0xffff0000u);
+                    const float r1 = x[2 * e + 1] - __uint_as_float(__float_as_uint(x[2 * e + 1]) & 0xffff0000u);
+                    ll[e] = pack_bf16_trunc(r0, r1);
+                }
+                hi = make_uint4(hh[0], hh[1], hh[2], hh[3]);
+                qlo[k][sl] = __builtin_bit_cast(bf16x8_t, make_uint4(ll[0], ll[1], ll[2], ll[3]));
+            } else {
+                hi = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.q) + qrow + d0);
+            }
+            if (k == wave) s_q[(k * NSLAB + sl) * 64 + lane] = hi;
+        }
+    }
+
+    // A wave may meet no key of an early query: its maximum then stays the lowest finite value, against
+    // which masked scores (-inf) give P = 0, and which the merge weighs with 0.
+    float m_run[NU], m_thr[NU], l_run[NU];  // log2 units; the score that may raise m_run; this lane's sum of P
+    f32x4_t acc[NU][NT];
+#pragma unroll
+    for (int k = 0; k < NU; k++) {
+        m_run[k] = -__FLT_MAX__;
+        m_thr[k] = -INFINITY;
+        l_run[k] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[k][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    uint4* const slot = s_tile + wave * TL::SLOT;
+    const uint32_t slot_lds = lds_address(s_tile) + 16 * TL::SLOT * wave;
+    // A K row spans RC chunks: segments of 64 chunks repeat its swizzle every 4 rows, from one segment
+    // to the next but for rows of 32 chunks, which take two.
+    const uint32_t koff0 = 16 * TL::ksrc(lane), koff1 = SEG > 1 ? 16 * (TL::ksrc(64 + lane) - 64) : 0;
+    // Loads of one of the wave's pairs: off / bytes of its two blocks' tiles (0 bytes, which reads as
+    // zeros, past the list or for an invalid id).
+    struct Pair {
+        int64_t off[2];
+        uint32_t bytes[2];
+    };
+    int ids_v = -1;  // lane l: block l % 2 of the wave's step l / 2 of the current 32
+    auto pair_at = [&](int step) {
+        Pair p;
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const int id = __builtin_amdgcn_readlane(ids_v, 2 * (step & 31) + b);
+            p.off[b] = (static_cast<int64_t>(id >= 0 ? id : 0) * Hkv + kvh) * (TILE * ELT);
+            p.bytes[b] = id >= 0 ? TILE * ELT : 0;
+        }
+        return p;
+    };
+    auto issue = [&](const char* cache, bool is_v, const Pair& p) {
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+            lds_load_tile<SEG>(buffer_rsrc_words(cache + p.off[b], p.bytes[b]), is_v ? 16 * TL::vsrc(lane, b) : koff0,
+                               is_v ? 16 * TL::vsrc(lane, b) : koff1, slot_lds + 16 * (TL::base(0, b) + (is_v ? TL::K_CHUNKS : 0)));
+    };
+
+    for (int c0 = 0; c0 < nkb; c0 += KCH) {
+        const int nkc = min(KCH, nkb - c0);
+        const int npair = (nkc + 1) / 2;
+        const int kend = (c0 + nkc) * 16;
+        const int kend_lo = min(klim_lo, kend);
+        __syncthreads();  // the previous chunk's ids are no longer read
+        for (int i = tid; i < nkc + kPad; i += 64 * WAVES) {
+            int id = i < nkc ? table[c0 + i] : -1;
+            id = id < a.num_blocks ? id : -1;
+            s_ids[i] = id;
+            if constexpr (KV == PA_DTYPE_INT8) {
+                s_ksc[i] = id >= 0 ? a.k_scale[static_cast<int64_t>(id) * Hkv + kvh] : 0.0f;
+                const float vsc = id >= 0 ? a.v_scale[static_cast<int64_t>(id) * Hkv + kvh] : 0.0f;
+                const float lv = fmaxf(__log2f(vsc), kMinLog2VScale);
+                s_vlg[i] = lv;
+                s_vrc[i] = __builtin_amdgcn_exp2f(-lv);
+            }
+        }
+        __syncthreads();
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the loop counts its own loads only
+        // ids of steps st .. st + 31 (st a multiple of 32) of this wave
+        auto refill = [&](int st) {
+            const int j = 2 * wave + 2 * WAVES * (st + (lane >> 1)) + (lane & 1);
+            ids_v = j < nkc ? s_ids[j] : -1;
+        };
+        refill(0);
+        Pair nxt = pair_at(0);
+        issue(kc, false, nxt);
+        issue(vc, true, nxt);
+        for (int st = 0, jl = 2 * wave; jl < 2 * npair; st++, jl += 2 * WAVES) {
+            const int lb = c0 + jl;
+            const char* tk = reinterpret_cast<const char*>(slot + TL::base(0, kblk));
+            const char* tv = reinterpret_cast<const char*>(slot + TL::base(0, pblk));
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * SEG) : "memory");
+            float v[NU][8];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int r = krow0 + 4 * h;
+                bf16x8_t kop[NSLAB];
+#pragma unroll
+                for (int sl = 0; sl < NSLAB; sl++) {
+                    if constexpr (ELT == 2) {
+                        kop[sl] = k_operand(*reinterpret_cast<const KR*>(tk + TL::kpos(r, 4 * sl + q4) * 16));
+                    } else {
+                        const int cc = 2 * sl + (q4 >> 1);
+                        kop[sl] = k_operand(*reinterpret_cast<const KR*>(tk + TL::kpos(r, cc) * 16 + (q4 & 1) * 8));
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < NU; k++) {
+                    f32x4_t sacc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int sl = 0; sl < NSLAB; sl++) {
+                        const bf16x8_t qhi = __builtin_bit_cast(bf16x8_t, s_q[(k * NSLAB + sl) * 64 + lane]);
+                        sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop[sl], qhi, sacc, 0, 0, 0);
+                        if constexpr (QF32) sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop[sl], qlo[k][sl], sacc, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; i++) v[k][4 * h + i] = sacc[i];
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (((st + 1) & 31) == 0) refill(st + 1);
+            nxt = pair_at(st + 1);
+            issue(kc, false, nxt);
+            if constexpr (KV == PA_DTYPE_INT8) {
+                const float mult = c2 * s_ksc[jl + pblk];
+                const float lvb = s_vlg[jl + pblk];
+#pragma unroll
+                for (int k = 0; k < NU; k++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[k][e] = __builtin_fmaf(v[k][e], mult, lvb);
+            }
+            if ((lb + 2) * 16 > kend_lo) {
+                const int kq = (lb + pblk) * 16 + ptok;
+#pragma unroll
+                for (int k = 0; k < NU; k++) {
+                    const int lim = min(causal ? P + i0[k] + n + 1 : T, kend) - kq;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[k][e] = e < lim ? v[k][e] : -INFINITY;
+                }
+            }
+            float bl[NU];
+            bool over = false;
+#pragma unroll
+            for (int k = 0; k < NU; k++) {
+                bl[k] = fmaxf(fmaxf(fmaxf(v[k][0], v[k][1]), fmaxf(v[k][2], v[k][3])),
+                              fmaxf(fmaxf(v[k][4], v[k][5]), fmaxf(v[k][6], v[k][7])));
+                over = over || bl[k] > m_thr[k];
+            }
+            if (__any(over)) {
+#pragma unroll
+                for (int k = 0; k < NU; k++) {
+                    float bm = rows_max(bl[k]);
+                    if constexpr (KV != PA_DTYPE_INT8) bm *= c2;
+                    const bool grow = bm > m_run[k] + kPrefillRescaleLog2;
+                    const float m_new = grow ? bm : m_run[k];
+                    const float alpha = __builtin_amdgcn_exp2f(m_run[k] - m_new);
+                    m_run[k] = m_new;
+                    m_thr[k] = KV != PA_DTYPE_INT8 ? (m_new + kPrefillRescaleLog2) / c2 : m_new + kPrefillRescaleLog2;
+                    l_run[k] *= alpha;
+                    float ar[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) ar[i] = __shfl(alpha, 4 * q4 + i, 64);
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[k][t][i] *= ar[i];
+                }
+            }
+            f16x8_t pf[NU];
+#pragma unroll
+            for (int k = 0; k < NU; k++) {
+                float p[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    if constexpr (KV == PA_DTYPE_INT8) p[e] = __builtin_amdgcn_exp2f(v[k][e] - m_run[k]);
+                    else p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[k][e], c2, -m_run[k]));
+                }
+                if constexpr (KV == PA_DTYPE_INT8) {
+                    const float rv = s_vrc[jl + pblk];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) l_run[k] = __builtin_fmaf(p[e], rv, l_run[k]);
+                }
+                uint32_t w[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const half2_t h = {static_cast<_Float16>(p[2 * e]), static_cast<_Float16>(p[2 * e + 1])};
+                    w[e] = __builtin_bit_cast(uint32_t, h);
+                    if constexpr (ELT == 2) l_run[k] = __builtin_amdgcn_fdot2(h, half2_t{1.0f, 1.0f}, l_run[k], false);
+                }
+                pf[k] = __builtin_bit_cast(f16x8_t, make_uint4(w[0], w[1], w[2], w[3]));
+            }
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * SEG) : "memory");
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const int d = 16 * t + n;
+                uint32_t o[4];
+                if constexpr (ELT == 2) {
+                    const uint4 x = *reinterpret_cast<const uint4*>(tv + TL::vpos(d, q4 >> 1, pblk) * 16);
+                    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const half2_t h = {static_cast<_Float16>(__uint_as_float(w[e] << 16)),
+                                           static_cast<_Float16>(__uint_as_float(w[e] & 0xffff0000u))};
+                        o[e] = __builtin_bit_cast(uint32_t, h);
+                    }
+                } else {
+                    const uint2 c = *reinterpret_cast<const uint2*>(tv + TL::vpos(d, 0, pblk) * 16 + (q4 >> 1) * 8);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint32_t x = e < 2 ? c.x : c.y;
+                        o[e] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(pa::i8_at(x, 2 * (e & 1)),
+                                                                                         pa::i8_at(x, 2 * (e & 1) + 1)));
+                    }
+                }
+                const f16x8_t vop = __builtin_bit_cast(f16x8_t, make_uint4(o[0], o[1], o[2], o[3]));
+#pragma unroll
+                for (int k = 0; k < NU; k++) acc[k][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf[k], vop, acc[k][t], 0, 0, 0);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(vc, true, nxt);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS-direct write outlives the chunk
+    }
+    __syncthreads();  // the rings are no longer read: they take the units' states
+
+    // The waves' states are added up through LDS, the sums brought to the larger maximum. State i of
+    // unit k: 16-byte word t of a lane at 64 t + lane.
+    auto leave = [&](int k, int i) {
+        uint4* st = s_tile + i * 64 * NST + lane;
+#pragma unroll
+        for (int t = 0; t < NT; t++) st[64 * t] = __builtin_bit_cast(uint4, acc[k][t]);
+        s_ml[i * 64 + lane] = make_float2(m_run[k], l_run[k]);
+    };
+    auto join = [&](int k, int i) {
+        const float2 ml = s_ml[i * 64 + lane];
+        const float mt = fmaxf(m_run[k], ml.x);
+        const float f0 = __builtin_amdgcn_exp2f(m_run[k] - mt), f1 = __builtin_amdgcn_exp2f(ml.x - mt);
+        m_run[k] = mt;
+        l_run[k] = l_run[k] * f0 + ml.y * f1;
+        float r0[4], r1[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            r0[e] = __shfl(f0, 4 * q4 + e, 64);
+            r1[e] = __shfl(f1, 4 * q4 + e, 64);
+        }
+        const uint4* st = s_tile + i * 64 * NST + lane;
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const f32x4_t x = __builtin_bit_cast(f32x4_t, st[64 * t]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[k][t][e] = acc[k][t][e] * r0[e] + x[e] * r1[e];
+        }
+    };
+    // Waves 4 .. 7 leave theirs to waves 0 .. 3, which then each end one unit. Waves past the last
+    // pair of blocks have none to leave.
+    const int busy = min(WAVES, (nkb + 1) / 2);
+    if (WAVES > 4 && busy > 4) {
+        if (wave >= 4 && wave < busy) {
+#pragma unroll
+            for (int k = 0; k < NU; k++) leave(k, NU * (wave - 4) + k);
+        }
+        __syncthreads();
+        if (wave < 4 && wave + 4 < busy) {
+#pragma unroll
+            for (int k = 0; k < NU; k++) join(k, NU * wave + k);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < NU; k++)
+        if (wave < 4 && wave < busy && k != wave) leave(k, 3 * k + (wave < k ? wave : wave - 1));
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NU; k++) {
+        if (k != wave) continue;
+#pragma unroll
+        for (int g = 0; g < 3; g++)
+            if (g + (g >= k) < busy) join(k, 3 * k + g);
+        const float l_tot = rows_sum(l_run[k]);  // query n's, in every lane of column n
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int qi = 4 * q4 + i;
+            if (qi < nq[k]) {
+                const float inv = 1.0f / __shfl(l_tot, qi, 64);
+                float* op = a.out + (static_cast<int64_t>(q0 + i0[k] + qi) * Hq + head[k]) * D;
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    if constexpr (ELT == 2) bad = bad || (__float_as_uint(acc[k][t][i]) & 0x7f800000u) == 0x7f800000u;
+                    op[16 * t + n] = acc[k][t][i] * inv;
+                }
+            }
+        }
+        if constexpr (ELT == 2) {
+            if (__any(bad))
+                prefill_exact_unit<D, QF32>(a, table, kvh, head[k], q0 + i0[k], nq[k], P + i0[k], T, causal);
+        }
+    }
+}
+
+template <int D, int KV, bool QF32>
+void launch(const PrefillArgs& a, bool wave, dim3 grid, hipStream_t s) {
+    using L = WaveLds<D, KV, QF32>;
+    static_assert(sizeof(L) <= 160 << 10, "the LDS of a CU");
+    if (wave) chunked_prefill_wave_kernel<D, KV, QF32><<<grid, 64 * L::WAVES, sizeof(L), s>>>(a);
+    else chunked_prefill_kernel<D, KV, QF32><<<grid, kPrefillThreads, 0, s>>>(a);
 }
 
 template <int D>
-void launch_kv(const PrefillArgs& a, int kv, bool qf32, dim3 grid, hipStream_t s) {
-    if (kv == PA_DTYPE_BF16) launch<D, PA_DTYPE_BF16>(a, qf32, grid, s);
-    else launch<D, PA_DTYPE_INT8>(a, qf32, grid, s);
+void launch_kv(const PrefillArgs& a, bool wave, int kv, bool qf32, dim3 grid, hipStream_t s) {
+    if (kv == PA_DTYPE_BF16) {
+        if (qf32) launch<D, PA_DTYPE_BF16, true>(a, wave, grid, s);
+        else launch<D, PA_DTYPE_BF16, false>(a, wave, grid, s);
+    } else {
+        if (qf32) launch<D, PA_DTYPE_INT8, true>(a, wave, grid, s);
+        else launch<D, PA_DTYPE_INT8, false>(a, wave, grid, s);
+    }
 }
 
 }  // namespace
@@ -799,19 +1283,30 @@ extern "C" pa_status pa_chunked_prefill(pa_stream* stream, const pa_config* cfg,
     a.mask_mode = mask_mode;
     a.scale = pa::resolve_scale(cfg);
 
-    a.qtiles_per_wg = a.group >= pa::kPrefillUnits ? 1 : pa::kPrefillUnits / a.group;
-    a.num_qgroups = ((max_chunk_len + 15) / 16 + a.qtiles_per_wg - 1) / a.qtiles_per_wg;
     const int64_t ng = static_cast<int64_t>(num_seqs) * cfg->num_kv_heads;
-    const int64_t nwg = static_cast<int64_t>(a.num_qgroups) * ((ng + 7) / 8) * 8;
+    const int64_t tiles = (static_cast<int64_t>(max_chunk_len) + 15) / 16;
+    // Calls whose workgroups the wave-split kernel runs in one generation (one a CU) go to it when
+    // there may be keys to split (256: 13.0 against 13.6 us without a prefix, 19.9 against 16.3 with 256
+    // tokens), calls of one and a half to two generations when the context may reach 1024 tokens
+    // (2 x 512 on 800 tokens 43.7 against 40.6 us; 1024 on 2000 88 against 64.5; three generations: 54
+    // against 59). The table's width bounds the context; the prefix lengths are on the device.
+    const int units = pa::wave_units(cfg->head_dim);
+    const int64_t wave_wgs = (tiles * a.group + units - 1) / units;
+    const int64_t cus = pa::device_cus(), w = ng * wave_wgs;
+    bool wave = (w <= cus && max_blocks_per_seq >= 16) || (2 * w > 3 * cus && w <= 2 * cus && max_blocks_per_seq >= 64);
+    a.qtiles_per_wg = a.group >= pa::kPrefillUnits ? 1 : pa::kPrefillUnits / a.group;
+    const int64_t qgroups = wave ? wave_wgs : (tiles + a.qtiles_per_wg - 1) / a.qtiles_per_wg;
+    a.num_qgroups = static_cast<int32_t>(qgroups);
+    const int64_t nwg = wave ? (ng / 8 * qgroups + (ng % 8 * qgroups + 7) / 8) * 8 : qgroups * ((ng + 7) / 8) * 8;
     if (nwg > 0x7fffffff) return pa::set_error(PA_ERROR_UNSUPPORTED, "pa_chunked_prefill: grid too large");
     a.num_groups = static_cast<int32_t>(ng);
     const dim3 grid(static_cast<uint32_t>(nwg));
     hipStream_t s = pa::native(stream);
     const bool qf32 = cfg->q_dtype == PA_DTYPE_FP32;
     switch (cfg->head_dim) {
-        case 64: pa::launch_kv<64>(a, cfg->kv_dtype, qf32, grid, s); break;
-        case 128: pa::launch_kv<128>(a, cfg->kv_dtype, qf32, grid, s); break;
-        default: pa::launch_kv<256>(a, cfg->kv_dtype, qf32, grid, s); break;
+        case 64: pa::launch_kv<64>(a, wave, cfg->kv_dtype, qf32, grid, s); break;
+        case 128: pa::launch_kv<128>(a, wave, cfg->kv_dtype, qf32, grid, s); break;
+        default: pa::launch_kv<256>(a, wave, cfg->kv_dtype, qf32, grid, s); break;
     }
     PA_HIP_CHECK(hipGetLastError());
     return pa::clear_error();

@@ -199,3 +199,20 @@ def test_prefill_values_beyond_fp16_range(stream, flags, kv_dtype, q_dtype, Hq, 
     f = getattr(edit, "factor", 1.0)
     assert np.abs(ref).max() > 1000.0, "the case must reach large outputs"
     check_close(got / f, ref / f, **tol_for(kv_dtype), what=f"large V kv={kv_dtype} D={D} flags={flags} x{f}")
+
+
+@pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D,prefix,chunk", [
+    (1, 1, 8, 2, 128, [223, 0, 255, 16], [33, 1, 16, 250]),   # heads of a tile; queries some waves have no key for
+    (1, 0, 6, 2, 128, [300, 7], [17, 48]),                    # G = 3: units of a workgroup span two tiles
+    (1, 1, 4, 4, 64, [500, 0], [65, 64]),                     # G = 1: four tiles a workgroup
+    (1, 1, 2, 1, 64, [16370, 3], [18, 5]),                    # keys past 1024 blocks, a workgroup with one pair
+    (2, 0, 4, 1, 128, [8180, 0], [30, 40]),                   # int8 scales past 512 blocks
+    (2, 1, 16, 1, 64, [260, 9], [2, 31]),
+    (1, 1, 8, 1, 256, [400, 0], [40, 16]),
+    (2, 0, 2, 2, 256, [241, 270], [15, 1]),
+])
+def test_prefill_keys_split_over_waves(stream, kv_dtype, q_dtype, Hq, Hkv, D, prefix, chunk):
+    """Few workgroups and tables of 16 blocks or more: the waves of a workgroup split its keys."""
+    got, ref = run_prefill(stream, prefix=prefix, chunk=chunk, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=kv_dtype,
+                           q_dtype=q_dtype, seed=40 + D + Hq)
+    check_close(got, ref, **tol_for(kv_dtype), what=f"keys split over waves kv={kv_dtype} D={D} G={Hq // Hkv}")
