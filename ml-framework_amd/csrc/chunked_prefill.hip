@@ -848,22 +848,9 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>(
     int* const s_ids = sh.ids;
     float *const s_ksc = sh.ksc, *const s_vlg = sh.vlg, *const s_vrc = sh.vrc;
 
-    // Workgroup -> (sequence, KV head) group gi and unit group qg, the ones with the most keys first:
-    // as above every group runs on XCD gi mod 8, where its workgroups share its K/V in one L2, but for
-    // the last num_groups mod 8 groups, whose workgroups are dealt to the XCDs in equal runs.
-    const int qgs = a.num_qgroups, xcd = blockIdx.x & 7, whole = a.num_groups >> 3;
-    int wk = blockIdx.x >> 3, gi;
-    if (wk < whole * qgs) {
-        gi = xcd + 8 * (wk / qgs);
-        wk %= qgs;
-    } else {
-        const int rest = (a.num_groups & 7) * qgs, per = (rest + 7) >> 3;
-        const int j = xcd * per + wk - whole * qgs;
-        if (j >= rest) return;
-        gi = 8 * whole + j / qgs;
-        wk = j % qgs;
-    }
-    const int qg = qgs - 1 - wk;
+    int gi, wk;
+    if (!place_workgroup(a.num_groups, a.num_qgroups, gi, wk)) return;
+    const int qg = a.num_qgroups - 1 - wk;  // the ones with the most keys first
     const int seq = gi / a.num_kv_heads, kvh = gi - seq * a.num_kv_heads;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1297,7 +1284,7 @@ extern "C" pa_status pa_chunked_prefill(pa_stream* stream, const pa_config* cfg,
     a.qtiles_per_wg = a.group >= pa::kPrefillUnits ? 1 : pa::kPrefillUnits / a.group;
     const int64_t qgroups = wave ? wave_wgs : (tiles + a.qtiles_per_wg - 1) / a.qtiles_per_wg;
     a.num_qgroups = static_cast<int32_t>(qgroups);
-    const int64_t nwg = wave ? (ng / 8 * qgroups + (ng % 8 * qgroups + 7) / 8) * 8 : qgroups * ((ng + 7) / 8) * 8;
+    const int64_t nwg = wave ? pa::placed_grid(ng, qgroups) : qgroups * ((ng + 7) / 8) * 8;
     if (nwg > 0x7fffffff) return pa::set_error(PA_ERROR_UNSUPPORTED, "pa_chunked_prefill: grid too large");
     a.num_groups = static_cast<int32_t>(ng);
     const dim3 grid(static_cast<uint32_t>(nwg));

@@ -559,6 +559,30 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char*)p));  // generic -> LDS offset
 }
 
+// Placement of the prefills' workgroups, `per` of them for each of num_groups (sequence, KV head)
+// groups. Workgroup ids are dispatched to the 8 XCDs in turn: group gi runs on XCD gi mod 8, where
+// its workgroups share its K/V in one L2, but for the last num_groups mod 8 groups, whose workgroups are
+// dealt to the XCDs in equal runs (2 groups would otherwise leave 6 XCDs idle). Gives the group and
+// the workgroup's place in it; false for an id past the last.
+__device__ __forceinline__ bool place_workgroup(int num_groups, int per, int& gi, int& wk) {
+    const int xcd = blockIdx.x & 7, whole = num_groups >> 3;
+    wk = blockIdx.x >> 3;
+    if (wk < whole * per) {
+        gi = xcd + 8 * (wk / per);
+        wk %= per;
+        return true;
+    }
+    const int rest = (num_groups & 7) * per, run = (rest + 7) >> 3;
+    const int j = xcd * run + wk - whole * per;
+    if (j >= rest) return false;
+    gi = 8 * whole + j / per;
+    wk = j % per;
+    return true;
+}
+inline int64_t placed_grid(int64_t num_groups, int64_t per) {
+    return (num_groups / 8 * per + (num_groups % 8 * per + 7) / 8) * 8;
+}
+
 // ---- launchers (one translation unit per kernel family) ----------------------------------------
 constexpr int kMaxPersistentSeqs = 2048;  // per-sequence tables of the persistent kernel (LDS)
 constexpr int kMaxDecodeWorkers = 4096;   // workers (waves) of one MFMA decode launch, at most

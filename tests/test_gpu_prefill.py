@@ -216,3 +216,19 @@ def test_prefill_keys_split_over_waves(stream, kv_dtype, q_dtype, Hq, Hkv, D, pr
     got, ref = run_prefill(stream, prefix=prefix, chunk=chunk, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=kv_dtype,
                            q_dtype=q_dtype, seed=40 + D + Hq)
     check_close(got, ref, **tol_for(kv_dtype), what=f"keys split over waves kv={kv_dtype} D={D} G={Hq // Hkv}")
+
+
+@pytest.mark.parametrize("q_dtype,Hq,Hkv,D,prefix,chunk", [
+    (0, 6, 2, 64, [333, 0], [17, 1]),                          # an odd number of units; one unit a wave
+    (1, 1, 1, 128, [16 * 64 * 8 - 3, 0], [3, 16]),             # more than 64 blocks a wave
+    (0, 8, 8, 64, [100, 0, 31], [130, 305, 16]),               # two units a wave, eight waves on their keys
+    (0, 16, 16, 32, [0, 20, 300, 7, 0], [150, 260, 16, 1, 250]),  # four
+    (1, 8, 8, 32, [5] * 15 + [200], [400] * 15 + [391]),       # two
+    (0, 9, 3, 32, [0] * 40, [481] + [353] * 39),               # one
+    (0, 4, 2, 256, [70, 0, 300], [33, 16, 120]),
+])
+def test_prefill_fp32_waves_per_unit(stream, q_dtype, Hq, Hkv, D, prefix, chunk):
+    """fp32 caches: every number of waves that share a unit's keys, units that pair up or stand alone."""
+    got, ref = run_prefill(stream, prefix=prefix, chunk=chunk, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=0, q_dtype=q_dtype,
+                           seed=60 + D + Hq)
+    check_close(got, ref, **tol_for(0), what=f"fp32 waves per unit D={D} G={Hq // Hkv} S={len(prefix)}")
