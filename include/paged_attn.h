@@ -211,9 +211,9 @@ pa_status pa_build_slot_mapping(pa_stream* stream, const pa_config* cfg,
  *   (src/MLFramework/Quantization/Operations/QuantizationOperations.cs:188-200).
  *   A block's new tokens may sit anywhere in the call's token list (split by other blocks'
  *   tokens or invalid slots); its segments (maximal runs of them) are applied in call order.
- *   The int8 append scans the slot list once per touched block (a workgroup per block finds
- *   whether an earlier token of the call owns its block), so its cost grows as blocks x n_tok:
- *   prompts above about 16k tokens are best appended in calls of at most that many tokens.
+ *   The int8 append scans the slot list once per touched block (to find whether another token of
+ *   the call lands in it), so its cost grows as blocks x n_tok: prompts above about 16k tokens are
+ *   best appended in calls of at most that many tokens.
  *   k_scale/v_scale/k_absmax/v_absmax are required for INT8 and ignored otherwise. */
 pa_status pa_kv_append(pa_stream* stream, const pa_config* cfg,
                        const void* k_new, const void* v_new,

@@ -9,8 +9,8 @@
 // requantises every row it does not overwrite; the segment's rows are then quantised with the
 // block's (possibly grown) scale.
 //
-// Ownership: one workgroup per token of the call; the workgroup of the first token of the call
-// that lands in a block owns that block and applies every segment of it, in call order, one wave
+// Runs: a block whose tokens of the call are one run of consecutive slots takes append_int8_run.
+// Ownership, otherwise: the workgroup of the first token of the call that lands in a block owns that block and applies every segment of it, in call order, one wave
 // per (KV head, K|V). A block's tokens may therefore arrive in any order, split by invalid slots
 // or by other blocks' tokens, without two workgroups touching one block.
 #pragma once
@@ -229,6 +229,156 @@ __device__ __forceinline__ void append_int8_one_token(const float (&x)[D / 64], 
     }
 }
 
+// A run of m <= 16 consecutive slots (rows r0 .. r0 + m - 1 of block blk, tokens s .. s + m - 1) that are the
+// call's only tokens of their block, appended by one wave for (KV head h, K or V): the bytes and
+// statistics of append_int8_apply with that segment. All of the run's values are loaded at once and
+// held in registers between the maximum and the quantisation (token by token, as append_int8_apply
+// takes a segment of any length, a prompt's block waits for 32 round trips), lane = (row of a pass, 8
+// dims). K codes go out as 8-byte pieces of their rows; V codes are turned into [dim][row] through
+// `stage` (16 D bytes of LDS), 4 dims x D / 16 rows a lane, and merged with the rows that are kept. K
+// and V share the code: run once per wave, it is bound by its own fetch when unrolled for both
+// (17 us where this form takes 14). Sources are 16-byte aligned.
+template <int D, bool IN_BF16>
+__device__ __forceinline__ void append_int8_run(const void* src, int64_t tok_stride, int32_t s, int m, int r0,
+                                                int64_t blk, int8_t* cache, float* scale, float* absmax, int h,
+                                                int32_t num_kv_heads, bool is_v, int8_t* stage) {
+#pragma clang fp contract(off)
+    constexpr int kRows = 512 / D;             // rows of one pass, D / 8 lanes each
+    constexpr int kPasses = kBlockSize / kRows;
+    constexpr int kVRows = D / 16;             // V: rows of a lane (4 dims each), 256 / D lanes per 4 dims
+    const int lane = threadIdx.x & 63;
+    const int64_t sidx = blk * num_kv_heads + h;
+    int8_t* tile = cache + sidx * kBlockSize * D;
+    const bool fresh = r0 == 0;
+    const int c = lane % (D / 8);                 // the lane's 8 dims of a row
+    const int g = lane % (D / 4), vr = lane / (D / 4) * kVRows;  // V: its 4 dims and first row
+    // One round trip: the statistics, the tile's codes where they may be needed (requantised when the
+    // scale grows; V keeps the rows that are not written), the run's values. Old codes of K: 8 bytes of
+    // each pass; of V: kVRows bytes of each of the 4 dims.
+    const float amax_mem = fresh ? 0.0f : absmax[sidx];
+    const float scale_mem = fresh ? 0.0f : scale[sidx];
+    constexpr int kOld = kPasses * 2;  // words: the same number for V
+    static_assert(kOld == kVRows, "4 dims of kVRows / 4 words");
+    uint32_t old[kOld];
+#pragma unroll
+    for (int i = 0; i < kOld; i++) old[i] = 0;
+    if (!is_v && !fresh) {
+#pragma unroll
+        for (int p = 0; p < kPasses; p++) {
+            const uint2 w = *reinterpret_cast<const uint2*>(tile + (p * kRows + lane / (D / 8)) * D + 8 * c);
+            old[2 * p] = w.x;
+            old[2 * p + 1] = w.y;
+        }
+    } else if (is_v && (!fresh || m < kBlockSize)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int k = 0; k < kVRows / 4; k++)
+                old[e * (kVRows / 4) + k] = *reinterpret_cast<const uint32_t*>(tile + (4 * g + e) * kBlockSize + vr + 4 * k);
+    }
+    float x[kPasses * 8];
+    {
+        const int64_t base = static_cast<int64_t>(s) * tok_stride + static_cast<int64_t>(h) * D + 8 * c;
+        constexpr int kWords = IN_BF16 ? 1 : 2;
+        uint4 raw[kPasses][kWords];
+#pragma unroll
+        for (int p = 0; p < kPasses; p++) {
+            // rows outside the run read one of its rows: no new maximum, and their codes are not used
+            const int j = min(max(p * kRows + lane / (D / 8) - r0, 0), m - 1);
+            const char* at = static_cast<const char*>(src) + (base + j * tok_stride) * (IN_BF16 ? 2 : 4);
+#pragma unroll
+            for (int w = 0; w < kWords; w++) raw[p][w] = reinterpret_cast<const uint4*>(at)[w];
+        }
+#pragma unroll
+        for (int p = 0; p < kPasses; p++) {
+            const uint32_t w0[4] = {raw[p][0].x, raw[p][0].y, raw[p][0].z, raw[p][0].w};
+            const uint4 hi = raw[p][kWords - 1];
+            const uint32_t w1[4] = {hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if constexpr (IN_BF16) x[8 * p + e] = (e & 1) ? bf16_hi(w0[e >> 1]) : bf16_lo(w0[e >> 1]);
+                else x[8 * p + e] = __uint_as_float(e < 4 ? w0[e] : w1[e - 4]);
+            }
+        }
+    }
+    float seg_amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kPasses * 8; i++) {
+        const float a = fabsf(x[i]);
+        seg_amax = a > seg_amax ? a : seg_amax;  // NaN never wins, as `if (a > m) m = a`
+    }
+    seg_amax = wave_max_dpp(seg_amax);
+    const bool grow = !fresh && seg_amax > amax_mem;
+    const float cur_scale = fresh || grow ? seg_amax / 127.0f : scale_mem;
+    if (grow) {
+        // QuantizeSymmetric(Dequantize(q, old scale), new scale) of every old code
+#pragma unroll
+        for (int i = 0; i < kOld; i++) {
+            uint32_t w = old[i], o = 0;
+#pragma unroll 1
+            for (int b = 0; b < 4; b++) {
+                const float deq = static_cast<float>(static_cast<int8_t>(w & 0xffu)) * scale_mem;
+                o = (o >> 8) | (static_cast<uint32_t>(static_cast<uint8_t>(quantize_symmetric(deq, cur_scale))) << 24);
+                w >>= 8;
+            }
+            old[i] = o;
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < kPasses; p++) {
+        if ((p + 1) * kRows <= r0 && (is_v || !grow)) continue;  // a pass without a row of the run
+        if (p * kRows >= r0 + m && (is_v || !grow)) continue;
+        const int r = p * kRows + lane / (D / 8);
+        uint32_t o[2] = {0, 0};
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            o[e >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(quantize_symmetric(x[8 * p + e], cur_scale))) << (8 * (e & 3));
+        const bool in = r >= r0 && r < r0 + m;
+        if (is_v) *reinterpret_cast<uint2*>(stage + r * D + 8 * c) = make_uint2(o[0], o[1]);
+        else if (in || grow)
+            *reinterpret_cast<uint2*>(tile + r * D + 8 * c) = in ? make_uint2(o[0], o[1]) : make_uint2(old[2 * p], old[2 * p + 1]);
+    }
+    if (is_v) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's codes are in LDS
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < kVRows / 4; k++) {
+            // rows vr + 4 k .. + 3 of dims 4 g .. + 3: a 4 x 4 byte transpose
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] = *reinterpret_cast<const uint32_t*>(stage + (vr + 4 * k + i) * D + 4 * g);
+            const uint32_t a = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u), b = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
+            const uint32_t e = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u), f = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+            const uint32_t t[4] = {__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(b, a, 0x07060302u),
+                                   __builtin_amdgcn_perm(f, e, 0x05040100u), __builtin_amdgcn_perm(f, e, 0x07060302u)};
+            uint32_t keep = 0;  // bytes of rows outside the run
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int r = vr + 4 * k + i;
+                keep |= r >= r0 && r < r0 + m ? 0u : 0xffu << (8 * i);
+            }
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                uint32_t& o = old[d * (kVRows / 4) + k];
+                o = (o & keep) | (t[d] & ~keep);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            int8_t* at = tile + (4 * g + d) * kBlockSize + vr;
+            const uint32_t* o = old + d * (kVRows / 4);
+            if constexpr (kVRows == 4) *reinterpret_cast<uint32_t*>(at) = o[0];
+            else if constexpr (kVRows == 8) *reinterpret_cast<uint2*>(at) = make_uint2(o[0], o[1]);
+            else *reinterpret_cast<uint4*>(at) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+        __builtin_amdgcn_wave_barrier();  // the stage is written again by the wave's next run
+    }
+    if ((fresh || grow) && lane == 0) {
+        absmax[sidx] = seg_amax;
+        scale[sidx] = cur_scale;
+    }
+}
+
 // Segments collected per pass of the owner's scan (a block has at most 16 rows, so more than one
 // pass only happens when slots repeat).
 constexpr int kAppendSegList = 64;
@@ -243,7 +393,8 @@ inline int append_int8_threads(int32_t num_kv_heads) {
 // skipped when none of them lands in the block).
 constexpr int kAppendCoarse = 8;
 
-// The workgroup of token i (blockDim.x a multiple of 64, at most kAppendMaxThreads): if token i
+// The workgroup of token i (blockDim.x a multiple of 64, at most kAppendMaxThreads; `parts`
+// workgroups of one token share its (KV head, K|V) pairs, this one being `part`): if token i
 // is the first token of the call that lands in its block, applies every segment of that block, in
 // call order; otherwise returns. The owner reads the call's slot list once, kAppendCoarse slots per
 // thread at a time, and looks closer only at chunks that hold tokens of its block: a call of n
@@ -254,7 +405,7 @@ __device__ __forceinline__ void append_int8_block(const void* k_src, const void*
                                                   int64_t tok_stride, SlotAt slot_at, int32_t i, int32_t n_tok,
                                                   int8_t* k_cache, int8_t* v_cache, float* k_scale, float* v_scale,
                                                   float* k_absmax, float* v_absmax, int32_t num_kv_heads,
-                                                  int64_t capacity) {
+                                                  int64_t capacity, int32_t part = 0, int32_t parts = 1) {
     __shared__ int s_start[kAppendSegList], s_end[kAppendSegList];
     __shared__ int s_wcnt[2][kAppendMaxThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -331,7 +482,7 @@ __device__ __forceinline__ void append_int8_block(const void* k_src, const void*
             }
         }
         // Apply the complete segments, in order, one wave per (KV head, K|V).
-        for (int p = wave; p < 2 * num_kv_heads; p += nwaves) {
+        for (int p = part * nwaves + wave; p < 2 * num_kv_heads; p += parts * nwaves) {
             const int h = p >> 1;
             const bool is_v = (p & 1) != 0;
             float amax = 0.0f, cur_scale = 0.0f;

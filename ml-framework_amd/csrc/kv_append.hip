@@ -266,6 +266,104 @@ __global__ __launch_bounds__(pa::kAppendMaxThreads) void append_int8_kernel(
                              v_absmax, num_kv_heads, capacity);
 }
 
+// int8 caches with 16-byte aligned operands: gridDim.y workgroups of up to kRunWaves waves per W
+// consecutive tokens of the call, a wave per (KV head, K|V). A token that starts a run of consecutive
+// slots of one block, when no other token of the call lands in that block (a prompt chunk's blocks, a
+// decode's tokens), has the run appended from registers (append_int8_run); a block whose tokens come in
+// any other way is left to append_int8_block, its (KV head, K|V) pairs shared by the workgroups. One
+// pass over the call's slots looks for other tokens of all the blocks that start here.
+//
+// Latency-bound: slots, the look for other tokens and the run are three dependent round trips.
+// append_int8_block alone, a workgroup a token, takes a block's tokens one by one: 2048 tokens of 8 KV
+// heads of 128 in four chunks 64 us against 14.2 here, 16000 tokens 2270 against 79. W = 16 for calls
+// past kRunTokens: with a workgroup a token, 15 of 16 of a prompt's only read its slots, and a CU holds
+// few enough that they queue (28 us). The runs of a window, one for a prompt but up to 16 for scattered
+// tokens, are dealt to kRunShares workgroups (1000 decode tokens 32 us, as before, against 50 with
+// one). W = 1 below, where every token may be a run of its own (128 decode tokens 8.7 -> 6.7 us).
+constexpr int kRunWaves = 4;
+constexpr int kRunTokens = 256;
+constexpr int kRunShares = 4;
+template <int D, bool IN_BF16, int W>
+__global__ __launch_bounds__(64 * kRunWaves) void append_int8_run_kernel(
+    const void* __restrict__ k_new, const void* __restrict__ v_new, const int64_t* __restrict__ slot_mapping,
+    int32_t n_tok, int8_t* __restrict__ k_cache, int8_t* __restrict__ v_cache, float* __restrict__ k_scale,
+    float* __restrict__ v_scale, float* __restrict__ k_absmax, float* __restrict__ v_absmax, int32_t num_kv_heads,
+    int64_t capacity, int64_t tok_stride) {
+    __shared__ int s_blk[W], s_len[W], s_other;
+    __shared__ __align__(16) int8_t s_stage[kRunWaves][pa::kBlockSize * D];
+    const int i0 = blockIdx.x * W;
+    const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Lane l: token i0 - 1 + l's block (-1: none, skipped) and row, and whether it starts a segment of its block.
+    const int64_t u = static_cast<int64_t>(i0) - 1 + lane;
+    const int64_t sl = u >= 0 && u < n_tok ? slot_mapping[u] : -1;
+    const int blk = sl >= 0 && sl < capacity ? static_cast<int>(sl >> 4) : -1, row = static_cast<int>(sl & 15);
+    const int prev = __shfl_up(blk, 1, 64);
+    const uint64_t starts = __ballot(lane >= 1 && lane <= W && blk >= 0 && prev != blk);
+    // The starts of a window are dealt to gridDim.z workgroups.
+    uint64_t mine = 0;
+    int rank = 0;
+    for (uint64_t left = starts; left != 0; left &= left - 1, rank++)
+        if (rank % static_cast<int>(gridDim.z) == static_cast<int>(blockIdx.z)) mine |= left & -left;
+    if (mine == 0) return;
+    // Token i0 + w, if it starts a segment: its block and the length of its run of consecutive slots.
+    uint64_t filter = 0;
+    for (uint64_t left = mine; left != 0; left &= left - 1) {
+        const int l = __builtin_ctzll(left);
+        const int b = __builtin_amdgcn_readlane(blk, l), r = __builtin_amdgcn_readlane(row, l);
+        const uint64_t run = __ballot(blk == b && row == r + (lane - l)) >> l;
+        filter |= 1ull << (b & 63);
+        if (tid == 0) {
+            s_blk[l - 1] = b;
+            s_len[l - 1] = __builtin_ctzll(~run);  // at most 16: the run stays in its block
+        }
+    }
+    if (tid == 0) s_other = 0;
+    __syncthreads();
+    // Bit w of s_other: another token of the call lands in the block that starts at token i0 + w. Slots whose
+    // block's low six bits no such block has are passed over at once.
+    for (int t0 = 0; t0 < n_tok; t0 += pa::kAppendCoarse * nthreads) {
+        int64_t o[pa::kAppendCoarse];
+#pragma unroll
+        for (int k = 0; k < pa::kAppendCoarse; k++) {
+            const int t = t0 + k * nthreads + tid;
+            o[k] = t < n_tok ? slot_mapping[t] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < pa::kAppendCoarse; k++) {
+            if (o[k] < 0 || o[k] >= capacity) continue;
+            const int b = static_cast<int>(o[k] >> 4), t = t0 + k * nthreads + tid;
+            if (!((filter >> (b & 63)) & 1)) continue;
+            for (uint64_t left = mine; left != 0; left &= left - 1) {
+                const int w = __builtin_ctzll(left) - 1;
+                if (b == s_blk[w] && (t < i0 + w || t >= i0 + w + s_len[w])) atomicOr(&s_other, 1 << w);
+            }
+        }
+    }
+    __syncthreads();
+    const int others = s_other;
+    for (uint64_t left = mine; left != 0; left &= left - 1) {
+        const int l = __builtin_ctzll(left);
+        const int i = i0 + l - 1;
+        if ((others >> (l - 1)) & 1) {
+            pa::append_int8_block<D>(k_new, v_new, IN_BF16, tok_stride, [&](int t) { return slot_mapping[t]; }, i, n_tok,
+                                     k_cache, v_cache, k_scale, v_scale, k_absmax, v_absmax, num_kv_heads, capacity,
+                                     static_cast<int32_t>(blockIdx.y), static_cast<int32_t>(gridDim.y));
+            __syncthreads();  // its LDS is used again
+            continue;
+        }
+        const int b = __builtin_amdgcn_readlane(blk, l), r0 = __builtin_amdgcn_readlane(row, l);
+        const int len = __builtin_amdgcn_readfirstlane(s_len[l - 1]);
+        for (int p = static_cast<int>(blockIdx.y) * (nthreads >> 6) + wave; p < 2 * num_kv_heads;
+             p += static_cast<int>(gridDim.y) * (nthreads >> 6)) {
+            const bool v = (p & 1) != 0;
+            pa::append_int8_run<D, IN_BF16>(v ? v_new : k_new, tok_stride, i, len, r0, b, v ? v_cache : k_cache,
+                                            v ? v_scale : k_scale, v ? v_absmax : k_absmax, p >> 1, num_kv_heads, v,
+                                            s_stage[wave]);
+        }
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -341,6 +439,28 @@ pa_status launch_kv_append(const char* f, hipStream_t s, const pa_config* cfg, c
         const int threads = append_int8_threads(cfg->num_kv_heads);
         auto* kc = static_cast<int8_t*>(k_cache);
         auto* vc = static_cast<int8_t*>(v_cache);
+        if (aligned) {
+            const int tasks = 2 * cfg->num_kv_heads, waves = tasks < kRunWaves ? tasks : kRunWaves;
+            const int ny = (tasks + waves - 1) / waves;
+            const bool wide = n_tok > kRunTokens;
+            const dim3 grid(wide ? (n_tok + 15) / 16 : n_tok, ny < 65535 ? ny : 65535, wide ? kRunShares : 1);
+            auto go = [&](auto kern) {
+                kern<<<grid, 64 * waves, 0, s>>>(k_new, v_new, slot_mapping, n_tok, kc, vc, k_scale, v_scale, k_absmax,
+                                                 v_absmax, cfg->num_kv_heads, capacity, tok_stride);
+            };
+            switch (cfg->head_dim) {
+#define PA_APPEND_RUN(DD)                                                                                     \
+    if (wide) go(in_bf16 ? append_int8_run_kernel<DD, true, 16> : append_int8_run_kernel<DD, false, 16>);       \
+    else go(in_bf16 ? append_int8_run_kernel<DD, true, 1> : append_int8_run_kernel<DD, false, 1>);            \
+    break;
+                case 64: PA_APPEND_RUN(64)
+                case 128: PA_APPEND_RUN(128)
+                default: PA_APPEND_RUN(256)
+#undef PA_APPEND_RUN
+            }
+            PA_HIP_CHECK(hipGetLastError());
+            return clear_error();
+        }
         switch (cfg->head_dim) {
             case 64:
                 append_int8_kernel<64><<<n_tok, threads, 0, s>>>(k_new, v_new, in_bf16, slot_mapping, n_tok, kc, vc,

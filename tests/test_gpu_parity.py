@@ -265,6 +265,50 @@ def test_append_int8_bit_exact(stream, D, q_dtype):
     step(slots, k, v)
 
 
+@pytest.mark.parametrize("D,q_dtype,hkv", [(128, 0, 3), (64, 1, 1), (256, 1, 2), (128, 1, 8)])
+def test_append_int8_runs_bit_exact(stream, D, q_dtype, hkv):
+    """Runs of consecutive slots, each the call's only tokens of its block: short calls (a workgroup
+    per token) and calls past 256 tokens (a window of 16 tokens per workgroup), runs that start or end
+    inside a block, grow its scale or not, beside scattered tokens, invalid slots and blocks whose tokens
+    come in two parts, which leave the run path."""
+    rng = np.random.default_rng(190 + D + hkv)
+    nb = 60
+    cfg = pa.make_config(num_q_heads=hkv, num_kv_heads=hkv, head_dim=D, kv_dtype=2, q_dtype=q_dtype,
+                         num_blocks=nb)
+    host = dict(kc=np.zeros((nb, hkv, 16, D), np.int8), vc=np.zeros((nb, hkv, 16, D), np.int8),
+                ks=np.zeros((nb, hkv), np.float32), vs=np.zeros((nb, hkv), np.float32),
+                ka=np.zeros((nb, hkv), np.float32), va=np.zeros((nb, hkv), np.float32))
+    dev = {n: to_gpu(a) for n, a in host.items()}
+
+    def step(slots, mult=1.0):
+        slots = np.asarray(slots, np.int64)
+        k = (rng.standard_normal((len(slots), hkv, D), dtype=np.float32) * np.float32(mult)).astype(np.float32)
+        v = (rng.standard_normal((len(slots), hkv, D), dtype=np.float32) / np.float32(mult)).astype(np.float32)
+        v[len(slots) // 2] = np.nan if mult > 1 else 0.0
+        if q_dtype == 1:
+            k, v = orc.bf16_from_f32(k), orc.bf16_from_f32(v)
+        orc.kv_append(cfg, k, v, slots, host["kc"], host["vc"], host["ks"], host["vs"], host["ka"], host["va"])
+        pa.kv_append(stream, cfg, to_gpu(k), to_gpu(v), to_gpu(slots), len(slots), dev["kc"], dev["vc"],
+                     dev["ks"], dev["vs"], dev["ka"], dev["va"])
+        _sync()
+        for n, a in host.items():
+            np.testing.assert_array_equal(to_np(dev[n]), a, err_msg=n)
+
+    def run(block, row, n):
+        return np.arange(n) + block * 16 + row
+
+    perm = rng.permutation(nb)
+    step(run(3, 0, 5))                                              # a block's first rows
+    step(np.concatenate([run(3, 5, 4), run(9, 0, 16), run(7, 0, 1)]))
+    step(np.concatenate([run(3, 9, 7), [-1], run(7, 1, 3), [nb * 16], run(9, 2, 1)]), 3.0)  # growing scales
+    step(run(3, 4, 3), 0.25)                                        # rows rewritten within the scale
+    step(np.concatenate([run(b, 0, 16) for b in perm[:17]]))          # 272 tokens, whole blocks out of order
+    step(np.concatenate([run(perm[20], 3, 13)] + [run(b, 0, 16) for b in perm[21:40]] + [run(perm[40], 0, 9)]), 2.0)
+    # scattered single tokens, a padded stretch, a block in two parts, one in reverse order
+    step(np.concatenate([perm * 16 + rng.integers(0, 16, nb), np.full(40, -1), run(perm[1], 0, 5), run(perm[2], 0, 16),
+                         run(perm[1], 9, 4), run(perm[3], 0, 16)[::-1], np.concatenate([run(b, 0, 16) for b in perm[45:]])]), 1.5)
+
+
 @pytest.mark.parametrize("D,q_dtype", [(128, 0), (64, 1), (256, 0)])
 def test_append_int8_out_of_order_bit_exact(stream, D, q_dtype):
     """A block's tokens split by -1 padding, revisited after other blocks' tokens, a slot written
