@@ -603,6 +603,13 @@ extern template void launch_decode_mfma<32>(DecodeArgs&, int, bool, bool, bool, 
 extern template void launch_decode_mfma<64>(DecodeArgs&, int, bool, bool, bool, int, int64_t, hipStream_t);
 extern template void launch_decode_mfma<128>(DecodeArgs&, int, bool, bool, bool, int, int64_t, hipStream_t);
 extern template void launch_decode_mfma<256>(DecodeArgs&, int, bool, bool, bool, int, int64_t, hipStream_t);
+// bf16 / int8 caches, head_dim up to 128, contexts of at most kRowMaxLen tokens: one launch, no workspace.
+constexpr int kRowMaxLen = 16 * 64;  // a lane per block id
+template <int D>
+void launch_decode_row(const DecodeArgs& a, int kv_dtype, bool q_f32, bool append, int num_seqs, hipStream_t s);
+extern template void launch_decode_row<32>(const DecodeArgs&, int, bool, bool, int, hipStream_t);
+extern template void launch_decode_row<64>(const DecodeArgs&, int, bool, bool, int, hipStream_t);
+extern template void launch_decode_row<128>(const DecodeArgs&, int, bool, bool, int, hipStream_t);
 // fp32 caches: grid (max_parts, Hkv, num_seqs); returns false for an uncompiled shape.
 bool launch_decode_fp32(const DecodeArgs& a, int head_dim, dim3 grid, hipStream_t s);
 

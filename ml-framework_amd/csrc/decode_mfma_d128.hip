@@ -2,3 +2,4 @@
 #include "decode_mfma_launch.h"
 
 template void pa::launch_decode_mfma<128>(pa::DecodeArgs&, int, bool, bool, bool, int, int64_t, hipStream_t);
+template void pa::launch_decode_row<128>(const pa::DecodeArgs&, int, bool, bool, int, hipStream_t);

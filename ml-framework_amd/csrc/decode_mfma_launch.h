@@ -55,4 +55,28 @@ void launch_decode_mfma(DecodeArgs& a, int kv_dtype, bool q_f32, bool append, bo
     }
 }
 
+template <int D, int KV, bool QF32>
+void launch_row(const DecodeArgs& a, bool append, int num_seqs, hipStream_t s) {
+    const dim3 grid(a.num_kv_heads, num_seqs);
+    const size_t lds = static_cast<size_t>(kRowWaves) * a.group * (D + 2) * sizeof(float);  // the waves' (O, max, sum)
+    if constexpr (KV == PA_DTYPE_BF16) {
+        if (append) {
+            paged_decode_mfma_row_kernel<D, KV, QF32, true><<<grid, 64 * kRowWaves, lds, s>>>(a);
+            return;
+        }
+    }
+    paged_decode_mfma_row_kernel<D, KV, QF32, false><<<grid, 64 * kRowWaves, lds, s>>>(a);
+}
+
+template <int D>
+void launch_decode_row(const DecodeArgs& a, int kv_dtype, bool q_f32, bool append, int num_seqs, hipStream_t s) {
+    if (kv_dtype == PA_DTYPE_BF16) {
+        if (q_f32) launch_row<D, PA_DTYPE_BF16, true>(a, append, num_seqs, s);
+        else launch_row<D, PA_DTYPE_BF16, false>(a, append, num_seqs, s);
+    } else if constexpr (D >= 64) {  // int8 caches take no smaller head_dim (refused on the host)
+        if (q_f32) launch_row<D, PA_DTYPE_INT8, true>(a, append, num_seqs, s);
+        else launch_row<D, PA_DTYPE_INT8, false>(a, append, num_seqs, s);
+    }
+}
+
 }  // namespace pa

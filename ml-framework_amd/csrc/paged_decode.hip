@@ -336,6 +336,26 @@ pa_status decode_chunk(const char* fn, bool append, pa_stream* stream, const pa_
         PA_HIP_CHECK(hipGetLastError());
         append = false;  // the decode below reads the appended cache
     }
+    // Contexts of at most 1024 tokens, split by default: a workgroup per (sequence, KV head), except
+    //  - few rows with more than 512 tokens each (1 sequence of 1000 tokens, 8 KV heads: 14.2 against 12.8 us
+    //    over the whole chip; 4 such: 14.5 against 15.4);
+    //  - more than two rows a CU where they may be long and ragged (the longest is one workgroup's:
+    //    128 sequences of 30 to 1000, int8, 39.8 against 36.4 us; bf16, 35.3 against 36.7), or more than four
+    //    (256 sequences, bf16: 72 against 69 us of 333 tokens, 75 against 70 of 30 to 1000).
+    const int64_t nrows = static_cast<int64_t>(num_seqs) * cfg->num_kv_heads, cus = pa::device_cus();
+    const bool rows = part == 0 && cfg->num_splits == 0 && max_len <= pa::kRowMaxLen && cfg->head_dim <= 128 &&
+                      (max_len <= 512 || nrows >= 32) &&
+                      nrows <= (cfg->kv_dtype == PA_DTYPE_BF16 || max_len <= 512 ? 4 : 2) * cus;
+    if (rows) {
+        a.append_in_merge = 0;
+        switch (cfg->head_dim) {
+            case 32: pa::launch_decode_row<32>(a, cfg->kv_dtype, qf32, append, num_seqs, s); break;
+            case 64: pa::launch_decode_row<64>(a, cfg->kv_dtype, qf32, append, num_seqs, s); break;
+            default: pa::launch_decode_row<128>(a, cfg->kv_dtype, qf32, append, num_seqs, s); break;
+        }
+        PA_HIP_CHECK(hipGetLastError());
+        return pa::clear_error();
+    }
     switch (cfg->head_dim) {
         case 32: pa::launch_decode_mfma<32>(a, cfg->kv_dtype, qf32, append, false, num_seqs, max_grid, s); break;
         case 64: pa::launch_decode_mfma<64>(a, cfg->kv_dtype, qf32, append, false, num_seqs, max_grid, s); break;

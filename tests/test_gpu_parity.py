@@ -587,3 +587,26 @@ def test_decode_append_matches_append_then_decode(stream, kv_dtype, q_dtype, Hq,
         np.testing.assert_array_equal(to_np(ka), host_amax[0], err_msg="k_absmax")
         np.testing.assert_array_equal(to_np(va), host_amax[1], err_msg="v_absmax")
     check_close(to_np(out), ref, **tol_for(kv_dtype), what=f"fused append kv={kv_dtype} q={q_dtype} D={D}")
+
+
+# ---- short contexts: one workgroup per (sequence, KV head) --------------------------------------------
+# blocks per wave 1, 2, .. 16, waves without blocks, a new token that starts a block after each count
+ROW_LENS = [1, 2, 16, 17, 31, 33, 48, 49, 64, 65, 80, 81, 127, 129, 192, 193, 241, 255, 257, 385, 511, 513, 769, 960, 961,
+            1007, 1008, 1009, 1023, 1024]
+
+
+@pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D,lens", [
+    (1, 1, 32, 8, 128, ROW_LENS), (1, 0, 16, 1, 64, ROW_LENS + ROW_LENS), (1, 1, 4, 2, 32, ROW_LENS),
+    (2, 0, 32, 8, 128, ROW_LENS), (2, 1, 4, 4, 64, ROW_LENS), (1, 1, 32, 8, 128, [512]), (1, 0, 8, 8, 64, [497, 300]),
+])
+def test_decode_short_rows(stream, kv_dtype, q_dtype, Hq, Hkv, D, lens):
+    """Contexts of at most 1024 tokens, plain and fused, with a table wider than they need."""
+    w = wl.make_small(700 + D + kv_dtype, num_seqs=len(lens) + 1, lens=lens + [0], Hq=Hq, Hkv=Hkv, D=D, kv_dtype=kv_dtype,
+                      q_dtype=q_dtype)
+    wide = np.full((w.num_seqs, w.max_blocks + 9), -1, np.int32)
+    wide[:, :w.max_blocks] = w.block_tables
+    w.block_tables = wide
+    got, ref = run_decode(w, 65, stream)
+    check_close(got, ref, **tol_for(kv_dtype), what=f"short rows kv={kv_dtype} D={D} G={Hq // Hkv}")
+    assert np.all(got[-1] == 0.0)
+    test_decode_append_matches_append_then_decode(stream, kv_dtype, q_dtype, Hq, Hkv, D, 0, lens)
