@@ -141,3 +141,24 @@ def test_o_project_truncates_attention_output(n_tok):
     ref_r = orc.linear(orc.f32_from_bf16(base + 1), orc.f32_from_bf16(w))  # what rounding to nearest gives
     assert np.abs(ref_r - ref_t).max() > 3 * GEMM_RTOL * np.abs(ref_t).max()  # the case separates the two
     gemm_close(to_np(y), ref_t, "o gemm (truncation)")
+
+
+@pytest.mark.parametrize("hq,d,n_tok,shift", [(8, 64, 70, 1), (1, 32, 65, 0), (4, 128, 97, 3)])
+def test_o_project_bf16_copy(hq, d, n_tok, shift):
+    """The rocBLAS path's bf16 copy of the attention output, 16-byte aligned or not."""
+    import torch
+
+    rng = np.random.default_rng(32)
+    cfg = pa.make_config(num_q_heads=hq, num_kv_heads=1, head_dim=d, kv_dtype=1, q_dtype=1, num_blocks=4)
+    attn = rng.standard_normal((n_tok, hq, d), dtype=np.float32)
+    w = orc.bf16_from_f32(rng.standard_normal((64, hq * d), dtype=np.float32))
+    flat = empty_gpu((attn.size + shift,), np.float32)
+    flat[shift:] = to_gpu(attn.reshape(-1))
+    y = empty_gpu((n_tok, 64), np.float32)
+    wsb = pa.o_workspace_size(cfg, 64, n_tok)
+    ws = empty_gpu((wsb,), np.uint8)
+    pa.o_project(None, cfg, flat[shift:], to_gpu(w), 64, n_tok, y, ws, wsb)
+    torch.cuda.synchronize()
+    a16 = orc.bf16_from_f32(attn.reshape(n_tok, -1))
+    np.testing.assert_array_equal(to_np(ws)[:a16.nbytes].view(np.uint16).reshape(a16.shape), a16)
+    gemm_close(to_np(y), orc.linear(orc.f32_from_bf16(a16), orc.f32_from_bf16(w)), "o gemm")
