@@ -1112,14 +1112,17 @@ __global__ __launch_bounds__(64 * decode_waves(D), D > 128 ? 1 : 2) void paged_d
 // heads of 128, bf16, us before -> now: 1 sequence of 333 tokens 12.0 -> 7.4; 16 of 333, 15.3 -> 8.3; 64 of 30
 // to 1000, 25.5 -> 22.4; 128 of 333, 40.2 -> 31.2 (5.7 TB/s). Eight waves measured slower throughout (64 of
 // 90: 14.5 against 8.9; at 172 registers a wave a CU holds one such workgroup).
+//
+// The appended token is written value by value once the row has been streamed: sequences that share a
+// block and append different slots of it in one call must not rewrite each other's. A fifth wave for it
+// halved the workgroups a CU holds (128 of 333 tokens: 38 us).
 constexpr int kRowWaves = 4;
 
 template <int D, int KV, bool QF32, bool APPEND>
 __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kernel(const DecodeArgs a) {
     constexpr int WAVES = kRowWaves;
     constexpr int THREADS = 64 * WAVES;
-    __shared__ float s_app[APPEND ? 2 * D : 1];                 // the appended token's K and V values
-    __shared__ uint4 s_vtile[APPEND ? D * 16 * 2 / 16 : 1];     // and its V tile, both the owning wave's
+    __shared__ float s_app[APPEND ? 2 * D : 1];  // the appended token's K and V values, the owning wave's
     extern __shared__ float s_part[];
     const int kvh = blockIdx.x, seq = blockIdx.y;
     const int tid = threadIdx.x;
@@ -1160,6 +1163,17 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kerne
     b.ws_o = s_part;
     b.ws_m = s_part + WAVES * G * D;
     b.ws_l = b.ws_m + WAVES * G;
+    b.append_in_merge = 1;  // the owning wave only attends to the new token
+    // The new token's K (threads 0 .. D - 1) and V (D .. 2D - 1) values for the cache, one a thread.
+    uint16_t nbits = 0;
+    int nbid = -1;
+    if constexpr (APPEND) {
+        static_assert(2 * D <= THREADS, "a thread per value");
+        if (tid < 2 * D)
+            nbits = pa::bf16_trunc(act_at(tid < D ? a.k_new : a.v_new, !a.q_bf16,
+                                          (static_cast<int64_t>(seq) * Hkv + kvh) * D + (tid & (D - 1))));
+        nbid = valid_bid(a, __builtin_amdgcn_readlane(ids, ((T - 1) / 16) & 63));
+    }
     if (wave < busy) {
         const Piece g{seq, kvh, wave * c, min(nb, (wave + 1) * c), Ts, busy == 1 ? -1 : wave, true, 1};
         // lane j: block g.b0 + j (with the append one more, the block a new token at its row 0 starts)
@@ -1178,10 +1192,18 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kerne
             load_side<D, KV, QF32, APPEND, false>(b, g, my_ids, true, side);
         }
         const Piece none{};
-        mfma_piece<D, KV, QF32, APPEND, false>(b, g, my_ids, side, bufs, st, s_app, s_vtile, false, none, -1, nside, [] {});
+        mfma_piece<D, KV, QF32, APPEND, false>(b, g, my_ids, side, bufs, st, s_app, nullptr, false, none, -1, nside, [] {});
+    }
+    if (busy > 1) __syncthreads();
+    if constexpr (APPEND) {
+        if (tid < 2 * D && nbid >= 0) {
+            const int64_t tile = (static_cast<int64_t>(nbid) * Hkv + kvh) * 16 * D;
+            const int at = (T - 1) & 15, d = tid & (D - 1);
+            if (tid < D) __builtin_nontemporal_store(nbits, static_cast<uint16_t*>(const_cast<void*>(a.k_cache)) + tile + at * D + d);
+            else __builtin_nontemporal_store(nbits, static_cast<uint16_t*>(const_cast<void*>(a.v_cache)) + tile + d * 16 + at);
+        }
     }
     if (busy == 1) return;
-    __syncthreads();
     for (int idx = tid; idx < G * D; idx += THREADS) {
         const int g = idx / D;
         float m[WAVES], mt = -INFINITY;

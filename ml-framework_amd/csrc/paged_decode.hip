@@ -347,7 +347,6 @@ pa_status decode_chunk(const char* fn, bool append, pa_stream* stream, const pa_
                       (max_len <= 512 || nrows >= 32) &&
                       nrows <= (cfg->kv_dtype == PA_DTYPE_BF16 || max_len <= 512 ? 4 : 2) * cus;
     if (rows) {
-        a.append_in_merge = 0;
         switch (cfg->head_dim) {
             case 32: pa::launch_decode_row<32>(a, cfg->kv_dtype, qf32, append, num_seqs, s); break;
             case 64: pa::launch_decode_row<64>(a, cfg->kv_dtype, qf32, append, num_seqs, s); break;

@@ -610,3 +610,31 @@ def test_decode_short_rows(stream, kv_dtype, q_dtype, Hq, Hkv, D, lens):
     check_close(got, ref, **tol_for(kv_dtype), what=f"short rows kv={kv_dtype} D={D} G={Hq // Hkv}")
     assert np.all(got[-1] == 0.0)
     test_decode_append_matches_append_then_decode(stream, kv_dtype, q_dtype, Hq, Hkv, D, 0, lens)
+
+
+@pytest.mark.parametrize("D,base", [(32, 0), (64, 16), (128, 160)])
+def test_decode_append_shared_last_block(stream, D, base):
+    """16 sequences append the 16 slots of one block in one call: the
+    cache holds every token (what each attends to of the others' is not defined, so not compared)."""
+    S, Hkv = 16, 4
+    w = wl.make_small(900 + D, num_seqs=S, lens=[base + 1 + i for i in range(S)], Hq=8, Hkv=Hkv, D=D, kv_dtype=1, q_dtype=1)
+    w.block_tables = w.block_tables.copy()
+    w.block_tables[:, base // 16] = w.block_tables[0, base // 16]
+    inp = wl.numpy_inputs(w, 79)
+    cfg = config_for(w)
+    rng = np.random.default_rng(80)
+    k_new = orc.bf16_from_f32(rng.standard_normal((S, Hkv, D), dtype=np.float32))
+    v_new = orc.bf16_from_f32(rng.standard_normal((S, Hkv, D), dtype=np.float32))
+    pos = w.context_lens.astype(np.int64) - 1
+    slots = w.block_tables[np.arange(S), pos // 16].astype(np.int64) * 16 + pos % 16
+    kc, vc = to_gpu(inp["k_cache"]), to_gpu(inp["v_cache"])
+    hk, hv = inp["k_cache"].copy(), inp["v_cache"].copy()
+    orc.kv_append(cfg, k_new, v_new, slots, hk, hv)
+    out = empty_gpu((S, 8, D), np.float32)
+    wsb = pa.decode_workspace_size(cfg, S, w.max_context_len)
+    ws = empty_gpu((max(wsb, 1),), np.uint8)
+    pa.paged_decode_append(stream, cfg, out, to_gpu(inp["q"]), to_gpu(k_new), to_gpu(v_new), kc, vc, None, None, None,
+                           None, to_gpu(w.block_tables), to_gpu(w.context_lens), S, w.max_blocks, w.max_context_len, ws, wsb)
+    _sync()
+    np.testing.assert_array_equal(to_np(kc, np.uint16).reshape(hk.shape), hk)
+    np.testing.assert_array_equal(to_np(vc, np.uint16).reshape(hv.shape), hv)
