@@ -6,8 +6,13 @@ namespace {
 
 template <int D, int G>
 void launch_g(const DecodeArgs& a, dim3 grid, hipStream_t s) {
-    if (a.part == 512) paged_decode_fp32_kernel<D, G, 512><<<grid, 256, 0, s>>>(a);
-    else paged_decode_fp32_kernel<D, G, 256><<<grid, 256, 0, s>>>(a);
+    if constexpr (G >= 4) {  // a matrix step takes four heads
+        if (a.part == 512) paged_decode_fp32_mfma_kernel<D, G, 512><<<grid, 256, 0, s>>>(a);
+        else paged_decode_fp32_mfma_kernel<D, G, 256><<<grid, 256, 0, s>>>(a);
+    } else {
+        if (a.part == 512) paged_decode_fp32_kernel<D, G, 512><<<grid, 256, 0, s>>>(a);
+        else paged_decode_fp32_kernel<D, G, 256><<<grid, 256, 0, s>>>(a);
+    }
 }
 
 template <int D>

@@ -589,6 +589,23 @@ def test_decode_append_matches_append_then_decode(stream, kv_dtype, q_dtype, Hq,
     check_close(to_np(out), ref, **tol_for(kv_dtype), what=f"fused append kv={kv_dtype} q={q_dtype} D={D}")
 
 
+@pytest.mark.parametrize("part", [0, 512])
+@pytest.mark.parametrize("q_dtype,Hq,Hkv,D", [(0, 8, 2, 32), (1, 8, 1, 32), (0, 16, 2, 64), (1, 4, 1, 64), (0, 8, 2, 128),
+                                              (0, 16, 2, 128), (1, 8, 2, 256), (0, 8, 1, 256)])
+def test_decode_fp32_grouped_heads(stream, part, q_dtype, Hq, Hkv, D):
+    """fp32 caches, groups of 4 and 8 heads (matrix kernel): partitions with 0 to 4 (8) blocks a wave and
+    every kind of last block, a block outside the cache (zeros), wide tables, no context."""
+    lens = [0, 1, 3, 4, 15, 16, 17, 48, 49, 64, 65, 127, 240, 256, 257, 300, 511, 512, 513, 1100]
+    w = wl.make_small(950 + D + Hq, num_seqs=len(lens), lens=lens, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=0, q_dtype=q_dtype)
+    wide = np.full((w.num_seqs, w.max_blocks + 3), -1, np.int32)
+    wide[:, :w.max_blocks] = w.block_tables
+    wide[13, 2] = -1
+    w.block_tables = wide
+    got, ref = run_decode(w, 81, stream, partition_size=part)
+    check_close(got, ref, **tol_for(0), what=f"fp32 G={Hq // Hkv} D={D} part={part}")
+    assert np.all(got[0] == 0.0)
+
+
 # ---- short contexts: one workgroup per (sequence, KV head) --------------------------------------------
 # blocks per wave 1, 2, .. 16, waves without blocks, a new token that starts a block after each count
 ROW_LENS = [1, 2, 16, 17, 31, 33, 48, 49, 64, 65, 80, 81, 127, 129, 192, 193, 241, 255, 257, 385, 511, 513, 769, 960, 961,
