@@ -580,6 +580,10 @@ __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, 
         } else {
 #pragma unroll
             for (int u = 0; u < D / 32; u++) bf16_v_exchange(vr[2 * u], vr[2 * u + 1]);
+            // P as bf16 high and low parts. The low ones are rounded (one instruction a pair, as truncation
+            // is): truncated they leave every P short of the value that joined the sum, which all but the
+            // maximum's own blocks (P = 1) add up, so few long portions erred more than many short ones. Error
+            // of the output's norm against 64 bits, 64 sequences of 128 to 4096 tokens: 9.4e-6 truncated, 4.7e-6.
             uint32_t hi[2], lo[2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
@@ -587,7 +591,7 @@ __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, 
                 const float h0 = __uint_as_float(__float_as_uint(a0) & 0xffff0000u);
                 const float h1 = __uint_as_float(__float_as_uint(a1) & 0xffff0000u);
                 hi[e] = pack_bf16_trunc(a0, a1);
-                lo[e] = pack_bf16_trunc(a0 - h0, a1 - h1);
+                lo[e] = pack_bf16_rne(a0 - h0, a1 - h1);
             }
             const s16x4_t phi = __builtin_bit_cast(s16x4_t, make_uint2(hi[0], hi[1]));
             const s16x4_t plo = __builtin_bit_cast(s16x4_t, make_uint2(lo[0], lo[1]));
