@@ -335,9 +335,10 @@ __device__ __forceinline__ void bf16_v_exchange(uint2& x0, uint2& x1) {
 // previous piece, or for a worker's first piece by the worker), and it issues the next piece's
 // side loads at its start and its first two blocks in its last two iterations. prefetch_next() is
 // called once, after the piece's first loads, to start the id loads of the piece after the next.
-// s_new: this wave's LDS staging of the appended token (2 * D floats); s_vt: its V tile staging
-// (16 D bf16).
-template <int D, int KV, bool QF32, bool APPEND, bool SHARED, typename Prefetch>
+// s_new: this wave's LDS staging of the appended token (2 * D floats).
+// WRITES (with APPEND): the wave that owns a row's new token also writes it into the cache, unless
+// a.append_in_merge, through its V tile staged in s_vt (16 D bf16). Without, s_vt is not used.
+template <int D, int KV, bool QF32, bool APPEND, bool SHARED, bool WRITES, typename Prefetch>
 __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, int my_bid,
                                            PieceSide<D, QF32>& side, PipeBufs<D, KV>& bufs, RowState<D / 16>& st,
                                            float* s_new, uint4* s_vt, const bool& has_next, const Piece& nxt,
@@ -610,7 +611,7 @@ __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, 
     // held across the loop; a zero-sized descriptor for an invalid id writes zeros, never stored).
     int abid = -1;
     auto prefetch_vtile = [&]() {
-        if constexpr (APPEND) {
+        if constexpr (WRITES) {
             if (piece_owns_new<APPEND>(g) && !a.append_in_merge) {
                 if ((T & 15) != 0) {
                     abid = __builtin_amdgcn_readlane(my_bid, nb - 1);
@@ -727,14 +728,15 @@ __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, 
                 kx[e] = __uint_as_float(__float_as_uint(new_val(side.nk, e)) & 0xffff0000u);
                 vx[e] = __uint_as_float(__float_as_uint(new_val(side.nv, e)) & 0xffff0000u);
             }
-            uint16_t* vt16 = reinterpret_cast<uint16_t*>(s_vt);
             const int r = T & 15;
             if (lane * NPL < D) {
 #pragma unroll
                 for (int e = 0; e < NPL; e++) {
                     s_new[lane * NPL + e] = kx[e];
                     s_new[D + lane * NPL + e] = vx[e];
-                    vt16[(lane * NPL + e) * 16 + r] = static_cast<uint16_t>(__float_as_uint(vx[e]) >> 16);
+                    if constexpr (WRITES)
+                        reinterpret_cast<uint16_t*>(s_vt)[(lane * NPL + e) * 16 + r] =
+                            static_cast<uint16_t>(__float_as_uint(vx[e]) >> 16);
                 }
             }
             __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the stores have landed in LDS
@@ -772,7 +774,7 @@ __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, 
             }
             // The cache (unless the merge kernel writes the token): K row r as is, the V tile
             // (patched in LDS above) in full lines.
-            if (abid >= 0 && !a.append_in_merge) {
+            if (WRITES && abid >= 0 && !a.append_in_merge) {
                 const int64_t tile = (static_cast<int64_t>(abid) * Hkv + kvh) * TILE;
                 uint16_t* kc = static_cast<uint16_t*>(const_cast<void*>(a.k_cache)) + tile + r * D;
                 if (lane * NPL < D) {
@@ -1091,7 +1093,7 @@ __global__ __launch_bounds__(64 * decode_waves(D), D > 128 ? 1 : 2) void paged_d
         Piece nxt2;
         bool has_next2 = false;
         int nxt2_ids = -1;
-        mfma_piece<D, KV, QF32, APPEND, SHARED>(a, cur, cur_ids, side, bufs, st, s_new, s_vt, has_next, nxt,
+        mfma_piece<D, KV, QF32, APPEND, SHARED, APPEND>(a, cur, cur_ids, side, bufs, st, s_new, s_vt, has_next, nxt,
                                                 nxt_ids, nside, [&]() {
                                                     if (has_next) has_next2 = next_piece(nxt2);
                                                     if (has_next2) nxt2_ids = piece_ids_of<APPEND>(a, nxt2, lane);
@@ -1167,7 +1169,6 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kerne
     b.ws_o = s_part;
     b.ws_m = s_part + WAVES * G * D;
     b.ws_l = b.ws_m + WAVES * G;
-    b.append_in_merge = 1;  // the owning wave only attends to the new token
     // The new token's K (threads 0 .. D - 1) and V (D .. 2D - 1) values for the cache, one a thread.
     uint16_t nbits = 0;
     int nbid = -1;
@@ -1196,7 +1197,7 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kerne
             load_side<D, KV, QF32, APPEND, false>(b, g, my_ids, true, side);
         }
         const Piece none{};
-        mfma_piece<D, KV, QF32, APPEND, false>(b, g, my_ids, side, bufs, st, s_app, nullptr, false, none, -1, nside, [] {});
+        mfma_piece<D, KV, QF32, APPEND, false, false>(b, g, my_ids, side, bufs, st, s_app, nullptr, false, none, -1, nside, [] {});
     }
     if (busy > 1) __syncthreads();
     if constexpr (APPEND) {
