@@ -62,9 +62,9 @@ struct DecodeArgs {
     // MFMA kernel: > 0 cuts every row (sequence, KV head) into this many partitions of whole
     // blocks instead of the batch-wide equal ranges (pa_config.num_splits)
     int32_t num_splits;
-    // Fused append (bf16 caches) when the merge kernel runs: the decode folds the new token into
-    // attention from k_new / v_new and the merge kernel writes it into the cache.
-    int32_t append_in_merge;
+    // Fused append (bf16 caches): the decode folds the new token into attention from k_new / v_new,
+    // and a launch after it (the merge, or append_token_bf16_kernel) writes the token into the cache.
+    int32_t append_after;
 };
 
 
@@ -88,7 +88,7 @@ __device__ __forceinline__ float act_at(const void* p, bool f32, int64_t i) {
     return f32 ? static_cast<const float*>(p)[i] : pa::bf16_to_f32(static_cast<const uint16_t*>(p)[i]);
 }
 
-// The new token (position T - 1 of sequence seq, KV head kvh; T = its clamped context length >= 2)
+// The new token (position T - 1 of sequence seq, KV head kvh; T = its clamped context length >= 1)
 // written into a bf16 cache as pa_kv_append stores it: K row (T - 1) % 16 and V column (T - 1) % 16
 // of the block the table gives for it, bf16 by truncation. One wave, lane l takes dims l, l + 64, ..
 // Written by the merge kernel's fifth wave (beside the four merging ones, so its round trip is not
@@ -131,7 +131,7 @@ __device__ __forceinline__ void append_token_bf16_as(const DecodeArgs& a, int se
         ids[k] = whole_row && b < a.max_blocks_per_seq ? row[b] : -1;
     }
     const int T = clamp_len(a, a.context_lens[seq]);
-    if (T < 2) return;  // T == 1: the decode writes it (no streamed block); T <= 0: nothing
+    if (T < 1) return;
     const int bi = (T - 1) / 16;
     int bid;
     if (whole_row) {
@@ -160,6 +160,15 @@ template <int D>
 __device__ __forceinline__ void append_token_bf16(const DecodeArgs& a, int seq, int kvh) {
     if (a.q_bf16) append_token_bf16_as<D, false>(a, seq, kvh);
     else append_token_bf16_as<D, true>(a, seq, kvh);
+}
+
+// The new tokens of a fused append whose decode has no merge launch: a wave per (KV head, sequence).
+// They are written when every row has been read, so that sequences that share blocks (rows of one
+// table, a copy that has not been made yet) read what the cache held before the call, and not each
+// other's new tokens or parts of them by timing.
+template <int D>
+__global__ __launch_bounds__(64) void append_token_bf16_kernel(const DecodeArgs a) {
+    append_token_bf16<D>(a, blockIdx.y, blockIdx.x);
 }
 
 // Final write of one (sequence, query head, dim): normalised output, or the partition's partial.
@@ -373,14 +382,14 @@ __device__ __forceinline__ int64_t split_range_blocks(const DecodeArgs& a, int64
 // head, in unit u = w * Hkv + kvh: slot 2u, except range w1 when the sequence starts inside it (the
 // row is then that unit's last row portion, slot 2u + 1).
 // Launched with kMergeThreads threads, or kMergeThreads + 64 when it also writes the fused
-// append's token (a.append_in_merge): that fifth wave only writes the token.
+// append's token (a.append_after): that fifth wave only writes the token.
 constexpr int kMergeThreads = 256;
 template <int D>
 __global__ __launch_bounds__(kMergeThreads + 64) void paged_decode_merge_split_kernel(const DecodeArgs a,
                                                                                       int32_t num_seqs) {
     const int kvh = blockIdx.x, seq = blockIdx.y;
     if (threadIdx.x >= kMergeThreads) {
-        if (a.append_in_merge) append_token_bf16<D>(a, seq, kvh);
+        if (a.append_after) append_token_bf16<D>(a, seq, kvh);
         return;
     }
     const int64_t R0 = a.ws_pref[seq];

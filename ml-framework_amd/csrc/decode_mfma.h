@@ -26,7 +26,7 @@
 // the end of the row portion that holds the row's last streamed block. No block is patched in
 // registers, so the fused kernel streams with the same loop (and carry) as the plain decode. The
 // token is written into the cache by the split-merge kernel that follows the decode
-// (append_in_merge): written here, among the decode's reads, the V column (one line per dim of
+// (append_after): written here, among the decode's reads, the V column (one line per dim of
 // the tile) cost the step about 3 us whatever the form of the stores. Without a merge launch
 // (a single range) the owning wave writes it: its K row as is, its V column by rewriting the
 // whole V tile, fetched into LDS when the piece starts, patched there and stored back.
@@ -337,7 +337,7 @@ __device__ __forceinline__ void bf16_v_exchange(uint2& x0, uint2& x1) {
 // called once, after the piece's first loads, to start the id loads of the piece after the next.
 // s_new: this wave's LDS staging of the appended token (2 * D floats).
 // WRITES (with APPEND): the wave that owns a row's new token also writes it into the cache, unless
-// a.append_in_merge, through its V tile staged in s_vt (16 D bf16). Without, s_vt is not used.
+// a.append_after, through its V tile staged in s_vt (16 D bf16). Without, s_vt is not used.
 template <int D, int KV, bool QF32, bool APPEND, bool SHARED, bool WRITES, typename Prefetch>
 __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, int my_bid,
                                            PieceSide<D, QF32>& side, PipeBufs<D, KV>& bufs, RowState<D / 16>& st,
@@ -612,7 +612,7 @@ __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, 
     int abid = -1;
     auto prefetch_vtile = [&]() {
         if constexpr (WRITES) {
-            if (piece_owns_new<APPEND>(g) && !a.append_in_merge) {
+            if (piece_owns_new<APPEND>(g) && !a.append_after) {
                 if ((T & 15) != 0) {
                     abid = __builtin_amdgcn_readlane(my_bid, nb - 1);
                 } else if (nb < kPieceBlocks) {
@@ -774,7 +774,7 @@ __device__ __forceinline__ void mfma_piece(const DecodeArgs& a, const Piece& g, 
             }
             // The cache (unless the merge kernel writes the token): K row r as is, the V tile
             // (patched in LDS above) in full lines.
-            if (WRITES && abid >= 0 && !a.append_in_merge) {
+            if (WRITES && abid >= 0 && !a.append_after) {
                 const int64_t tile = (static_cast<int64_t>(abid) * Hkv + kvh) * TILE;
                 uint16_t* kc = static_cast<uint16_t*>(const_cast<void*>(a.k_cache)) + tile + r * D;
                 if (lane * NPL < D) {
@@ -1114,14 +1114,14 @@ __global__ __launch_bounds__(64 * decode_waves(D), D > 128 ? 1 : 2) void paged_d
 // What bounds a small decode is its chain of round trips. The persistent kernel above needs a prefix
 // over all context lengths, then block ids, then K/V, and a second launch that merges the ranges'
 // partials. Here the length, the row of the block table, Q and the new token are loaded together, so K/V
-// loads go out after one round trip, and nothing is written but the output. Fused append steps, 32 / 8
-// heads of 128, bf16, us before -> now: 1 sequence of 333 tokens 12.0 -> 7.4; 16 of 333, 15.3 -> 8.3; 64 of 30
-// to 1000, 25.5 -> 22.4; 128 of 333, 40.2 -> 31.2 (5.7 TB/s). Eight waves measured slower throughout (64 of
+// loads go out after one round trip, and no partial leaves the workgroup. Fused append steps, 32 / 8
+// heads of 128, bf16, us before -> now: 1 sequence of 333 tokens 12.6 -> 9.1 (calls
+// from Python, one after another); 16 of 333, 16.1 -> 11.7; 64 of 30 to 1000, 25.6 -> 24.9; 128 of 333, 38.7 -> 32.8. Eight waves measured slower throughout (64 of
 // 90: 14.5 against 8.9; at 172 registers a wave a CU holds one such workgroup).
 //
-// The appended token is written value by value once the row has been streamed: sequences that share a
-// block and append different slots of it in one call must not rewrite each other's. A fifth wave for it
-// halved the workgroups a CU holds (128 of 333 tokens: 38 us).
+// A call of one sequence writes its new token here, once the workgroup has streamed the row. With more
+// sequences (a.append_after) a row may hold a block that another appends to, so the tokens wait for a launch
+// of their own (append_token_bf16_kernel).
 constexpr int kRowWaves = 4;
 
 template <int D, int KV, bool QF32, bool APPEND>
@@ -1140,21 +1140,13 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kerne
     const int T = clamp_len(a, a.context_lens[seq]);  // with the new token
     float* const out = a.out + (static_cast<int64_t>(seq) * Hkv + kvh) * G * D;
     if (T <= (APPEND ? 1 : 0)) {
-        // No context: zeros. Fused append of a first token: its V (bf16 by truncation) in every head, and
-        // its K and V into row 0 of the sequence's first block.
+        // No context: zeros. Fused append of a first token: its V (bf16 by truncation) in every head.
         if (APPEND && T == 1) {
             const bool f32 = !a.q_bf16;
             const int64_t src = (static_cast<int64_t>(seq) * Hkv + kvh) * D;
             for (int idx = tid; idx < G * D; idx += THREADS)
                 out[idx] = __uint_as_float(__float_as_uint(act_at(a.v_new, f32, src + idx % D)) & 0xffff0000u);
-            const int bid = __builtin_amdgcn_readfirstlane(ids);
-            if (bid >= 0 && bid < a.num_blocks) {
-                const int64_t tile = (static_cast<int64_t>(bid) * Hkv + kvh) * 16 * D;
-                for (int d = tid; d < D; d += THREADS) {
-                    static_cast<uint16_t*>(const_cast<void*>(a.k_cache))[tile + d] = pa::bf16_trunc(act_at(a.k_new, f32, src + d));
-                    static_cast<uint16_t*>(const_cast<void*>(a.v_cache))[tile + d * 16] = pa::bf16_trunc(act_at(a.v_new, f32, src + d));
-                }
-            }
+            if (!a.append_after && wave == 0) append_token_bf16<D>(a, seq, kvh);
         } else {
             for (int idx = tid; idx < G * D; idx += THREADS) out[idx] = 0.0f;
         }
@@ -1174,10 +1166,12 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kerne
     int nbid = -1;
     if constexpr (APPEND) {
         static_assert(2 * D <= THREADS, "a thread per value");
-        if (tid < 2 * D)
-            nbits = pa::bf16_trunc(act_at(tid < D ? a.k_new : a.v_new, !a.q_bf16,
-                                          (static_cast<int64_t>(seq) * Hkv + kvh) * D + (tid & (D - 1))));
-        nbid = valid_bid(a, __builtin_amdgcn_readlane(ids, ((T - 1) / 16) & 63));
+        if (!a.append_after) {
+            if (tid < 2 * D)
+                nbits = pa::bf16_trunc(act_at(tid < D ? a.k_new : a.v_new, !a.q_bf16,
+                                              (static_cast<int64_t>(seq) * Hkv + kvh) * D + (tid & (D - 1))));
+            nbid = valid_bid(a, __builtin_amdgcn_readlane(ids, ((T - 1) / 16) & 63));
+        }
     }
     if (wave < busy) {
         const Piece g{seq, kvh, wave * c, min(nb, (wave + 1) * c), Ts, busy == 1 ? -1 : wave, true, 1};
@@ -1199,7 +1193,7 @@ __global__ __launch_bounds__(64 * kRowWaves, 2) void paged_decode_mfma_row_kerne
         const Piece none{};
         mfma_piece<D, KV, QF32, APPEND, false, false>(b, g, my_ids, side, bufs, st, s_app, nullptr, false, none, -1, nside, [] {});
     }
-    if (busy > 1) __syncthreads();
+    if (APPEND || busy > 1) __syncthreads();  // the row's blocks are read, the waves' partials written
     if constexpr (APPEND) {
         if (tid < 2 * D && nbid >= 0) {
             const int64_t tile = (static_cast<int64_t>(nbid) * Hkv + kvh) * 16 * D;

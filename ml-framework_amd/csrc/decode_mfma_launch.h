@@ -62,6 +62,7 @@ void launch_row(const DecodeArgs& a, bool append, int num_seqs, hipStream_t s) {
     if constexpr (KV == PA_DTYPE_BF16) {
         if (append) {
             paged_decode_mfma_row_kernel<D, KV, QF32, true><<<grid, 64 * kRowWaves, lds, s>>>(a);
+            if (a.append_after) append_token_bf16_kernel<D><<<grid, 64, 0, s>>>(a);
             return;
         }
     }

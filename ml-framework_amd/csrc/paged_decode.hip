@@ -325,7 +325,7 @@ pa_status decode_chunk(const char* fn, bool append, pa_stream* stream, const pa_
     // The merge kernel runs when there is more than one range (a row may span two); a fused bf16
     // append then has it write the new tokens into the cache.
     const bool merge = max_units > cfg->num_kv_heads;
-    a.append_in_merge = append && cfg->kv_dtype == PA_DTYPE_BF16 && merge ? 1 : 0;
+    a.append_after = append && cfg->kv_dtype == PA_DTYPE_BF16 && merge ? 1 : 0;
     if (append && cfg->kv_dtype == PA_DTYPE_INT8 && num_seqs > 0) {
         const int threads = pa::append_int8_threads(cfg->num_kv_heads);
         switch (cfg->head_dim) {
@@ -342,11 +342,21 @@ pa_status decode_chunk(const char* fn, bool append, pa_stream* stream, const pa_
     //  - more than two rows a CU where they may be long and ragged (the longest is one workgroup's:
     //    128 sequences of 30 to 1000, int8, 39.8 against 36.4 us; bf16, 35.3 against 36.7), or more than four
     //    (256 sequences, bf16: 72 against 69 us of 333 tokens, 75 against 70 of 30 to 1000).
+    // A bf16 append of several sequences takes a second launch, for the tokens: a row may hold the block that
+    // another sequence appends to. Against the persistent kernel and its merge, us, 8 KV heads of 128:
+    //  - 4 / 8 / 16 sequences of 1000 tokens 17.1 / 18.0 / 19.0 against 15.9 / 16.6 / 22.8: from one row for
+    //    two CUs on (8 of 30 to 1000: 14.3 against 16.0, given up);
+    //  - more than two rows a CU that may be long and ragged, as above (128 sequences of 30 to 1000: 39.3
+    //    against 36.6), or of 33 to 64 tokens, which are the persistent kernel's ranges one by one
+    //    (128 sequences of 60: 18.0 against 15.0; 64: 12.0 against 13.9; 128 of 32: 14.9 against 16.2).
+    const bool after = append && num_seqs > 1;
     const int64_t nrows = static_cast<int64_t>(num_seqs) * cfg->num_kv_heads, cus = pa::device_cus();
     const bool rows = part == 0 && cfg->num_splits == 0 && max_len <= pa::kRowMaxLen && cfg->head_dim <= 128 &&
-                      (max_len <= 512 || nrows >= 32) &&
-                      nrows <= (cfg->kv_dtype == PA_DTYPE_BF16 || max_len <= 512 ? 4 : 2) * cus;
+                      (max_len <= 512 || nrows >= (after ? cus / 2 : 32)) &&
+                      !(after && nrows > 2 * cus && max_len > 32 && max_len <= 64) &&
+                      nrows <= ((cfg->kv_dtype == PA_DTYPE_BF16 && !after) || max_len <= 512 ? 4 : 2) * cus;
     if (rows) {
+        a.append_after = after;
         switch (cfg->head_dim) {
             case 32: pa::launch_decode_row<32>(a, cfg->kv_dtype, qf32, append, num_seqs, s); break;
             case 64: pa::launch_decode_row<64>(a, cfg->kv_dtype, qf32, append, num_seqs, s); break;
@@ -364,7 +374,7 @@ pa_status decode_chunk(const char* fn, bool append, pa_stream* stream, const pa_
     PA_HIP_CHECK(hipGetLastError());
     if (merge) {
         dim3 mgrid(cfg->num_kv_heads, num_seqs);
-        const int mthreads = pa::kMergeThreads + (a.append_in_merge ? 64 : 0);
+        const int mthreads = pa::kMergeThreads + (a.append_after ? 64 : 0);
         switch (cfg->head_dim) {
             case 32: pa::paged_decode_merge_split_kernel<32><<<mgrid, mthreads, 0, s>>>(a, num_seqs); break;
             case 64: pa::paged_decode_merge_split_kernel<64><<<mgrid, mthreads, 0, s>>>(a, num_seqs); break;

@@ -631,8 +631,9 @@ def test_decode_short_rows(stream, kv_dtype, q_dtype, Hq, Hkv, D, lens):
 
 @pytest.mark.parametrize("D,base", [(32, 0), (64, 16), (128, 160)])
 def test_decode_append_shared_last_block(stream, D, base):
-    """16 sequences append the 16 slots of one block in one call: the
-    cache holds every token (what each attends to of the others' is not defined, so not compared)."""
+    """16 sequences append the 16 slots of one block in one call: the cache holds every token, and each
+    sequence attends to its own, and at the slots of the others that its context covers to what was there
+    before the call."""
     S, Hkv = 16, 4
     w = wl.make_small(900 + D, num_seqs=S, lens=[base + 1 + i for i in range(S)], Hq=8, Hkv=Hkv, D=D, kv_dtype=1, q_dtype=1)
     w.block_tables = w.block_tables.copy()
@@ -647,6 +648,12 @@ def test_decode_append_shared_last_block(stream, D, base):
     kc, vc = to_gpu(inp["k_cache"]), to_gpu(inp["v_cache"])
     hk, hv = inp["k_cache"].copy(), inp["v_cache"].copy()
     orc.kv_append(cfg, k_new, v_new, slots, hk, hv)
+    ref = np.empty((S, 8, D), np.float32)
+    for i in range(S):
+        own_k, own_v = inp["k_cache"].copy(), inp["v_cache"].copy()
+        orc.kv_append(cfg, k_new, v_new, np.where(np.arange(S) == i, slots, -1), own_k, own_v)
+        ref[i] = orc.paged_decode(cfg, inp["q"], own_k, own_v, None, None, w.block_tables, w.context_lens,
+                                  n_threads=NTHREADS)[i]
     out = empty_gpu((S, 8, D), np.float32)
     wsb = pa.decode_workspace_size(cfg, S, w.max_context_len)
     ws = empty_gpu((max(wsb, 1),), np.uint8)
@@ -655,3 +662,4 @@ def test_decode_append_shared_last_block(stream, D, base):
     _sync()
     np.testing.assert_array_equal(to_np(kc, np.uint16).reshape(hk.shape), hk)
     np.testing.assert_array_equal(to_np(vc, np.uint16).reshape(hv.shape), hv)
+    check_close(to_np(out), ref, **tol_for(1), what="shared block: every sequence's own new token only")
