@@ -253,9 +253,15 @@ pa_status pa_paged_decode(pa_stream* stream, const pa_config* cfg, float* out, c
  * pa_kv_append with slot_mapping[s] = block_tables[s][(T-1)/16] * 16 + (T-1) % 16 followed by
  * pa_paged_decode; for bf16 caches both happen in one kernel (the rows stream their first T - 1
  * cached tokens and the new token joins each row's softmax from k_new / v_new, truncated to bf16 as
- * the cache stores it, while the wave that ends the row writes it into the cache), for int8 caches the
+ * the cache stores it; it is written into the cache when every row has been read), for int8 caches the
  * quantising append is a launch of its own ahead of the decode, and for fp32 caches a plain
- * copy kernel. No reference counterpart: the reference appends (PagedAttentionLayer.UpdateKVCache,
+ * copy kernel.
+ * Sequences that share the block a token is appended to (rows of one table): every slot may be
+ * appended to once per call, and the cache ends up holding every token. Where the context of one
+ * sequence covers another's new slot, int8 and fp32 caches give it the new token; bf16 caches give it
+ * what the slot held before the call. (A call of more than 2047 sequences, 65535 for fp32 caches, is
+ * worked off as several calls of that many at most, in order.)
+ * No reference counterpart: the reference appends (PagedAttentionLayer.UpdateKVCache,
  * Layers/PagedAttentionLayer.cs:244-296) and decodes (DecodeOrchestrator.ComputeDecodeAttention,
  * Phases/DecodeOrchestrator.cs:64-80) in two steps; this is those two steps in one call.
  * Sequences with context_len <= 0 append nothing and produce zeros. */

@@ -28,8 +28,9 @@
 // token is written into the cache by the split-merge kernel that follows the decode
 // (append_after): written here, among the decode's reads, the V column (one line per dim of
 // the tile) cost the step about 3 us whatever the form of the stores. Without a merge launch
-// (a single range) the owning wave writes it: its K row as is, its V column by rewriting the
-// whole V tile, fetched into LDS when the piece starts, patched there and stored back.
+// (a single range) append_token_bf16_kernel writes it, or, in a call of one sequence, the owning wave:
+// its K row as is, its V column by rewriting the whole V tile, fetched into LDS when the piece starts,
+// patched there and stored back. Nothing is written while another sequence's row is read.
 //
 // Per block: S^T[16 tokens][16 heads] = K . Q^T on v_mfma_f32_16x16x32_bf16 (query heads padded
 // to 16 rows), online softmax in fp32, O[16 heads][D] += P . V on v_mfma_f32_16x16x16_bf16 with P
@@ -929,7 +930,7 @@ __global__ __launch_bounds__(64 * decode_waves(D), D > 128 ? 1 : 2) void paged_d
     const int Hkv = a.num_kv_heads;
     // Sequences with no context produce zeros. Fused append: a sequence whose only token is the new
     // one (context length 1) produces that token's V (bf16 by truncation) in every head of its KV
-    // head, and the token is written into row 0 of its first block.
+    // head, and the token is written into row 0 of its first block (unless a later launch does).
     for (int s = blockIdx.x; s < num_seqs; s += gridDim.x) {
         if (sh.lens[NG + s] > 0) continue;
         const int n = Hkv * a.group * D;
@@ -940,7 +941,7 @@ __global__ __launch_bounds__(64 * decode_waves(D), D > 128 ? 1 : 2) void paged_d
                 const float v = act_at(a.v_new, f32, (static_cast<int64_t>(s) * Hkv + kvh) * D + d);
                 a.out[static_cast<int64_t>(s) * n + idx] = __uint_as_float(__float_as_uint(v) & 0xffff0000u);
             }
-            const int bid = a.block_tables[static_cast<int64_t>(s) * a.max_blocks_per_seq];
+            const int bid = a.append_after ? -1 : a.block_tables[static_cast<int64_t>(s) * a.max_blocks_per_seq];
             if (bid >= 0 && bid < a.num_blocks) {
                 uint16_t* kc = static_cast<uint16_t*>(const_cast<void*>(a.k_cache));
                 uint16_t* vc = static_cast<uint16_t*>(const_cast<void*>(a.v_cache));

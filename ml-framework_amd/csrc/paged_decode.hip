@@ -323,9 +323,10 @@ pa_status decode_chunk(const char* fn, bool append, pa_stream* stream, const pa_
     const bool qf32 = cfg->q_dtype == PA_DTYPE_FP32;
     const int64_t max_grid = max_units > 0 ? max_units : 1;
     // The merge kernel runs when there is more than one range (a row may span two); a fused bf16
-    // append then has it write the new tokens into the cache.
+    // append then has it write the new tokens into the cache. With one range, the decode writes the token
+    // of a single sequence; those of several are written behind it, when every row has been read.
     const bool merge = max_units > cfg->num_kv_heads;
-    a.append_after = append && cfg->kv_dtype == PA_DTYPE_BF16 && merge ? 1 : 0;
+    a.append_after = append && cfg->kv_dtype == PA_DTYPE_BF16 && (merge || num_seqs > 1);
     if (append && cfg->kv_dtype == PA_DTYPE_INT8 && num_seqs > 0) {
         const int threads = pa::append_int8_threads(cfg->num_kv_heads);
         switch (cfg->head_dim) {
@@ -380,6 +381,15 @@ pa_status decode_chunk(const char* fn, bool append, pa_stream* stream, const pa_
             case 64: pa::paged_decode_merge_split_kernel<64><<<mgrid, mthreads, 0, s>>>(a, num_seqs); break;
             case 128: pa::paged_decode_merge_split_kernel<128><<<mgrid, mthreads, 0, s>>>(a, num_seqs); break;
             default: pa::paged_decode_merge_split_kernel<256><<<mgrid, mthreads, 0, s>>>(a, num_seqs); break;
+        }
+        PA_HIP_CHECK(hipGetLastError());
+    } else if (a.append_after) {
+        const dim3 tgrid(cfg->num_kv_heads, num_seqs);
+        switch (cfg->head_dim) {
+            case 32: pa::append_token_bf16_kernel<32><<<tgrid, 64, 0, s>>>(a); break;
+            case 64: pa::append_token_bf16_kernel<64><<<tgrid, 64, 0, s>>>(a); break;
+            case 128: pa::append_token_bf16_kernel<128><<<tgrid, 64, 0, s>>>(a); break;
+            default: pa::append_token_bf16_kernel<256><<<tgrid, 64, 0, s>>>(a); break;
         }
         PA_HIP_CHECK(hipGetLastError());
     }

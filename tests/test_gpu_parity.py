@@ -629,17 +629,21 @@ def test_decode_short_rows(stream, kv_dtype, q_dtype, Hq, Hkv, D, lens):
     test_decode_append_matches_append_then_decode(stream, kv_dtype, q_dtype, Hq, Hkv, D, 0, lens)
 
 
-@pytest.mark.parametrize("D,base", [(32, 0), (64, 16), (128, 160)])
-def test_decode_append_shared_last_block(stream, D, base):
-    """16 sequences append the 16 slots of one block in one call: the cache holds every token, and each
+@pytest.mark.parametrize("D,base,S,part", [
+    (32, 0, 16, 0), (64, 16, 16, 0), (128, 160, 16, 0),      # a workgroup per row
+    (64, 0, 16, 64), (128, 16, 16, 64), (256, 160, 16, 0),   # ranges and a merge; a first token among them
+    (256, 0, 4, 0), (128, 16, 2, 64),                        # one range, no merge
+])
+def test_decode_append_shared_last_block(stream, D, base, S, part):
+    """S sequences append slots 0 .. S - 1 of one block in one call: the cache holds every token, and each
     sequence attends to its own, and at the slots of the others that its context covers to what was there
     before the call."""
-    S, Hkv = 16, 4
+    Hkv = 4
     w = wl.make_small(900 + D, num_seqs=S, lens=[base + 1 + i for i in range(S)], Hq=8, Hkv=Hkv, D=D, kv_dtype=1, q_dtype=1)
     w.block_tables = w.block_tables.copy()
     w.block_tables[:, base // 16] = w.block_tables[0, base // 16]
     inp = wl.numpy_inputs(w, 79)
-    cfg = config_for(w)
+    cfg = config_for(w, partition_size=part)
     rng = np.random.default_rng(80)
     k_new = orc.bf16_from_f32(rng.standard_normal((S, Hkv, D), dtype=np.float32))
     v_new = orc.bf16_from_f32(rng.standard_normal((S, Hkv, D), dtype=np.float32))
