@@ -10,8 +10,9 @@
 // block's (possibly grown) scale.
 //
 // Runs: a block whose tokens of the call are one run of consecutive slots takes append_int8_run.
-// Ownership, otherwise: the workgroup of the first token of the call that lands in a block owns that block and applies every segment of it, in call order, one wave
-// per (KV head, K|V). A block's tokens may therefore arrive in any order, split by invalid slots
+// Ownership, otherwise: the workgroup of the first token of the call that lands in a block owns that
+// block and applies every segment of it, in call order, one wave per (KV head, K|V)
+// (append_int8_segments). A block's tokens may therefore arrive in any order, split by invalid slots
 // or by other blocks' tokens, without two workgroups touching one block.
 #pragma once
 
@@ -379,6 +380,190 @@ __device__ __forceinline__ void append_int8_run(const void* src, int64_t tok_str
     }
 }
 
+// Segments [starts[k], ends[k]), k < nseg (LDS), of block blk for (KV head h, K|V) by one wave: the bytes and
+// statistics of append_int8_apply called with each in turn. The tile's codes stay in registers from the
+// first segment to the last (lane l: the 16 rows of dims l, l + 64, ..), the absmax of up to 64 tokens is taken
+// before any is quantised, and their values are loaded kAhead tokens at a time. lut: 64 words of LDS. (Segment by segment each
+// waits for its values and its tile, and after a grown scale for the tile's stores: a block whose 16 tokens
+// come one by one, between other blocks' tokens, 55 us.)
+template <int D, typename SlotAt>
+__device__ __forceinline__ void append_int8_segments(const void* src, bool in_bf16, int64_t tok_stride,
+                                                     SlotAt slot_at, const int* starts, const int* ends, int nseg,
+                                                     int64_t blk, int8_t* cache, float* scale, float* absmax, int h,
+                                                     int32_t num_kv_heads, bool is_v, uint32_t* lut) {
+#pragma clang fp contract(off)
+    constexpr int kPer = D / 64, kAhead = 8;
+    const int lane = threadIdx.x & 63;
+    const int64_t sidx = blk * num_kv_heads + h;
+    int8_t* tile = cache + sidx * kBlockSize * D;
+    float amax = absmax[sidx], cur_scale = scale[sidx];
+    bool new_stats = false;
+    uint32_t dirty = 0;      // rows whose codes changed
+    uint32_t w[kPer][4];     // codes: byte r % 4 of word r / 4 is row r
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int d = lane + 64 * k;
+        if (is_v) {
+            const uint4 x = *reinterpret_cast<const uint4*>(tile + d * kBlockSize);
+            w[k][0] = x.x;
+            w[k][1] = x.y;
+            w[k][2] = x.z;
+            w[k][3] = x.w;
+        } else {
+            uint32_t b[kBlockSize];
+#pragma unroll
+            for (int r = 0; r < kBlockSize; r++) b[r] = static_cast<uint8_t>(tile[r * D + d]);
+#pragma unroll
+            for (int q = 0; q < 4; q++) w[k][q] = b[4 * q] | b[4 * q + 1] << 8 | b[4 * q + 2] << 16 | b[4 * q + 3] << 24;
+        }
+    }
+    auto load_token = [&](int t, float (&v)[kPer]) {
+        const int64_t base = static_cast<int64_t>(t) * tok_stride + static_cast<int64_t>(h) * D;
+#pragma unroll
+        for (int e = 0; e < kPer; e++) v[e] = load_act(src, in_bf16, base + lane + 64 * e);
+    };
+    auto token_max = [&](const float (&v)[kPer]) {
+        float m = 0.0f;
+#pragma unroll
+        for (int e = 0; e < kPer; e++) {
+            const float a = fabsf(v[e]);
+            m = a > m ? a : m;  // NaN never wins, as `if (a > m) m = a`
+        }
+        return m;
+    };
+    auto begin_segment = [&](bool fresh, float seg_amax) {
+        if (!fresh && !(seg_amax > amax)) return;
+        const float old_scale = cur_scale;
+        amax = seg_amax;
+        cur_scale = seg_amax / 127.0f;
+        new_stats = true;
+        if (fresh) return;
+        // QuantizeSymmetric(Dequantize(q, old scale), new scale) of every code, each of the 256 taken once (the
+        // lane's four; code by code a grown tile of head_dim 128 costs about 2 us); the segment's own rows are
+        // overwritten by its tokens.
+        dirty = (1u << kBlockSize) - 1;
+        uint32_t mine = 0;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const float deq = static_cast<float>(static_cast<int8_t>(4 * lane + b)) * old_scale;
+            mine |= static_cast<uint32_t>(static_cast<uint8_t>(quantize_symmetric(deq, cur_scale))) << (8 * b);
+        }
+        lut[lane] = mine;
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_wave_barrier();
+        const uint8_t* const to = reinterpret_cast<const uint8_t*>(lut);
+#pragma unroll
+        for (int e = 0; e < kPer; e++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t in = w[e][q];
+                w[e][q] = to[in & 0xffu] | to[in >> 8 & 0xffu] << 8 | to[in >> 16 & 0xffu] << 16 |
+                          static_cast<uint32_t>(to[in >> 24]) << 24;
+            }
+        __builtin_amdgcn_wave_barrier();  // the table is written again when the scale grows again
+    };
+    auto put = [&](int r, const float (&v)[kPer]) {
+        const uint32_t sh = 8 * (r & 3), keep = ~(0xffu << sh);
+        dirty |= 1u << r;
+#pragma unroll
+        for (int e = 0; e < kPer; e++) {
+            const uint32_t code = static_cast<uint32_t>(static_cast<uint8_t>(quantize_symmetric(v[e], cur_scale))) << sh;
+#pragma unroll
+            for (int q = 0; q < 4; q++) w[e][q] = (r >> 2) == q ? (w[e][q] & keep) | code : w[e][q];
+        }
+    };
+#pragma unroll 1
+    for (int k = 0; k < nseg;) {
+        // The next whole segments, up to 64 tokens: token of lane i, its row; the tokens that start a segment.
+        int tok = 0, cnt = 0;
+        uint64_t firsts = 0;
+        for (; k < nseg; k++) {
+            const int s = __builtin_amdgcn_readfirstlane(starts[k]);
+            const int len = __builtin_amdgcn_readfirstlane(ends[k]) - s;
+            if (cnt + len > 64) break;
+            if (lane >= cnt && lane < cnt + len) tok = s + lane - cnt;
+            firsts |= 1ull << cnt;
+            cnt += len;
+        }
+        if (cnt == 0) {  // a segment of more than 64 tokens: slots written several times; one after another
+            const int s = __builtin_amdgcn_readfirstlane(starts[k]), e = __builtin_amdgcn_readfirstlane(ends[k]);
+            bool fresh = false;
+            float m = 0.0f, v[kPer];
+            for (int t = s; t < e; t++) {
+                fresh = fresh || slot_at(t) % kBlockSize == 0;
+                load_token(t, v);
+                m = fmaxf(m, token_max(v));
+            }
+            begin_segment(fresh, wave_max_dpp(m));
+            for (int t = s; t < e; t++) {
+                load_token(t, v);
+                put(__builtin_amdgcn_readfirstlane(static_cast<int>(slot_at(t) % kBlockSize)), v);
+            }
+            k++;
+            continue;
+        }
+        const int row = lane < cnt ? static_cast<int>(slot_at(tok) % kBlockSize) : 0;
+        float x[kAhead][kPer];
+        auto load = [&](int i0) {
+#pragma unroll
+            for (int j = 0; j < kAhead; j++)
+                load_token(__builtin_amdgcn_readlane(tok, min(i0 + j, cnt - 1)), x[j]);
+        };
+        float tok_amax = 0.0f;  // lane i: token i's
+#pragma unroll 1
+        for (int i0 = 0; i0 < cnt; i0 += kAhead) {
+            load(i0);
+#pragma unroll
+            for (int j = 0; j < kAhead; j++) {
+                const float m = wave_max_dpp(token_max(x[j]));
+                tok_amax = lane == i0 + j ? m : tok_amax;
+            }
+        }
+#pragma unroll 1
+        for (int i0 = 0; i0 < cnt; i0 += kAhead) {
+            if (cnt > kAhead) load(i0);  // else still in x
+#pragma unroll 1
+            for (int j = 0; j < kAhead && i0 + j < cnt; j++) {
+                const int i = i0 + j;
+                float v[kPer];
+#pragma unroll
+                for (int e = 0; e < kPer; e++) {
+                    v[e] = x[0][e];
+#pragma unroll
+                    for (int q = 1; q < kAhead; q++) v[e] = j == q ? x[q][e] : v[e];
+                }
+                if (firsts >> i & 1) {
+                    const uint64_t later = firsts >> i >> 1;
+                    const int end = later != 0 ? i + 1 + __builtin_ctzll(later) : cnt;
+                    bool fresh = false;
+                    float seg_amax = 0.0f;
+                    for (int t = i; t < end; t++) {
+                        fresh = fresh || __builtin_amdgcn_readlane(row, t) == 0;
+                        seg_amax = fmaxf(seg_amax, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tok_amax), t)));
+                    }
+                    begin_segment(fresh, seg_amax);
+                }
+                put(__builtin_amdgcn_readlane(row, i), v);
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int d = lane + 64 * k;
+        if (is_v) {
+            if (dirty != 0) *reinterpret_cast<uint4*>(tile + d * kBlockSize) = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < kBlockSize; r++)
+                if (dirty >> r & 1) tile[r * D + d] = static_cast<int8_t>(w[k][r >> 2] >> (8 * (r & 3)));
+        }
+    }
+    if (new_stats && lane == 0) {
+        absmax[sidx] = amax;
+        scale[sidx] = cur_scale;
+    }
+}
+
 // Segments collected per pass of the owner's scan (a block has at most 16 rows, so more than one
 // pass only happens when slots repeat).
 constexpr int kAppendSegList = 64;
@@ -389,108 +574,104 @@ inline int append_int8_threads(int32_t num_kv_heads) {
     return static_cast<int>(64 * (waves < kAppendMaxThreads / 64 ? waves : kAppendMaxThreads / 64));
 }
 
-// Tokens per thread of the owner's coarse scan (a chunk of kAppendCoarse * blockDim.x tokens is
-// skipped when none of them lands in the block).
+// Tokens per thread of the scans over the call's slots.
 constexpr int kAppendCoarse = 8;
 
 // The workgroup of token i (blockDim.x a multiple of 64, at most kAppendMaxThreads; `parts`
 // workgroups of one token share its (KV head, K|V) pairs, this one being `part`): if token i
-// is the first token of the call that lands in its block, applies every segment of that block, in
-// call order; otherwise returns. The owner reads the call's slot list once, kAppendCoarse slots per
-// thread at a time, and looks closer only at chunks that hold tokens of its block: a call of n
-// tokens costs each touched block one pass over n slots (a few memory round trips for calls of up
-// to ~16k tokens; split much larger calls).
-template <int D, typename SlotAt>
+// is the first token of the call that lands in its block, or (OWNER) the caller has chosen it among
+// them, applies every segment of that block, in call order; otherwise returns. The owner reads the call's slot list once,
+// kAppendCoarse slots per thread at a time: a call of n tokens costs each touched block one pass over n
+// slots (a few memory round trips for calls of up to ~16k tokens; split much larger calls).
+template <int D, bool OWNER = false, typename SlotAt>
 __device__ __forceinline__ void append_int8_block(const void* k_src, const void* v_src, bool in_bf16,
                                                   int64_t tok_stride, SlotAt slot_at, int32_t i, int32_t n_tok,
                                                   int8_t* k_cache, int8_t* v_cache, float* k_scale, float* v_scale,
                                                   float* k_absmax, float* v_absmax, int32_t num_kv_heads,
                                                   int64_t capacity, int32_t part = 0, int32_t parts = 1) {
     __shared__ int s_start[kAppendSegList], s_end[kAppendSegList];
-    __shared__ int s_wcnt[2][kAppendMaxThreads / 64];
+    __shared__ int s_wcnt[kAppendMaxThreads / 64];
+    __shared__ uint32_t s_lut[kAppendMaxThreads / 64][64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nthreads = blockDim.x, nwaves = nthreads >> 6;
     auto valid = [&](int64_t sl) { return sl >= 0 && sl < capacity; };
     // Token i's slot and its predecessor's, loaded together.
     const int64_t slot_i = slot_at(i);
-    const int64_t slot_p = i > 0 ? slot_at(i - 1) : -1;
+    const int64_t slot_p = !OWNER && i > 0 ? slot_at(i - 1) : -1;
     if (!valid(slot_i)) return;
-    const int64_t blk = slot_i / kBlockSize;
+    const int64_t blk = __builtin_amdgcn_readfirstlane(static_cast<int>(slot_i / kBlockSize));
     if (valid(slot_p) && slot_p / kBlockSize == blk) return;  // not the first token of its segment
     auto in_blk = [&](int t) {
         if (t < 0 || t >= n_tok) return false;
         const int64_t sl = slot_at(t);
         return valid(sl) && sl / kBlockSize == blk;
     };
-    // Does any token of [lo, hi) land in the block? (coarse: kAppendCoarse tokens per thread)
-    auto any_in = [&](int lo, int hi) {
-        bool f = false;
-#pragma unroll
-        for (int k = 0; k < kAppendCoarse; k++) {
-            const int t = lo + k * nthreads + tid;
-            f |= t < hi && in_blk(t);
-        }
-        return __syncthreads_or(f) != 0;
-    };
     const int coarse = kAppendCoarse * nthreads;
-    // An earlier token of the call in the block: its workgroup owns the block.
-    for (int c0 = 0; c0 < i; c0 += coarse)
-        if (any_in(c0, i)) return;
+    if constexpr (!OWNER) {
+        // An earlier token of the call in the block: its workgroup owns the block.
+        for (int c0 = 0; c0 < i; c0 += coarse) {
+            bool f = false;
+#pragma unroll
+            for (int k = 0; k < kAppendCoarse; k++) {
+                const int t = c0 + k * nthreads + tid;
+                f |= t < i && in_blk(t);
+            }
+            if (__syncthreads_or(f)) return;
+        }
+    }
 
     // Passes: from seg_from on, segment starts and ends are compacted, in order, into s_start /
     // s_end until kAppendSegList segments are complete or the call ends; then they are applied.
-    int seg_from = i;
+    int seg_from = OWNER ? 0 : i;
     while (seg_from < n_tok) {
         int nseg = 0, nstart = 0;
         int resume = n_tok;  // where the next pass starts if this one fills the list
-        for (int c0 = seg_from; c0 < n_tok && resume == n_tok; c0 += coarse) {
-            if (!any_in(c0, n_tok)) continue;
-            const int c1 = min(n_tok, c0 + coarse);
-            for (int f0 = c0; f0 < c1; f0 += nthreads) {
-                const int t = f0 + tid;
-                const bool cur = t < c1 && in_blk(t);
-                const bool st = cur && !in_blk(t - 1);
-                const bool en = cur && !in_blk(t + 1);
-                const uint64_t ms = __ballot(st), me = __ballot(en);
-                const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-                if (lane == 0) {
-                    s_wcnt[0][wave] = __popcll(ms);
-                    s_wcnt[1][wave] = __popcll(me);
-                }
-                __syncthreads();
-                int bs = nstart, be = nseg, ts = 0, te = 0;
-                for (int w = 0; w < nwaves; w++) {
-                    if (w < wave) {
-                        bs += s_wcnt[0][w];
-                        be += s_wcnt[1][w];
-                    }
-                    ts += s_wcnt[0][w];
-                    te += s_wcnt[1][w];
-                }
-                const int rs = bs + __popcll(ms & below), re = be + __popcll(me & below);
-                if (st && rs < kAppendSegList) s_start[rs] = t;
-                if (en && re < kAppendSegList) s_end[re] = t + 1;
-                __syncthreads();
-                nstart += ts;
-                nseg += te;
-                if (nseg >= kAppendSegList) {
-                    nseg = kAppendSegList;
-                    resume = s_end[kAppendSegList - 1];
-                    break;
-                }
+        for (int c0 = seg_from; c0 < n_tok; c0 += coarse) {
+            // kAppendCoarse consecutive tokens a thread: bit j of `in`, token t0 - 1 + j lands in the block
+            const int t0 = c0 + kAppendCoarse * tid;
+            uint32_t in = 0;
+#pragma unroll
+            for (int j = 0; j < kAppendCoarse + 2; j++) in |= static_cast<uint32_t>(in_blk(t0 - 1 + j)) << j;
+            constexpr uint32_t kOwn = ((1u << kAppendCoarse) - 1) << 1;
+            const uint32_t starts = in & ~(in << 1) & kOwn, ends = in & ~(in >> 1) & kOwn;
+            // places in the lists: starts in the low half, ends in the high one
+            const int mine = __popc(starts) | __popc(ends) << 16;
+            int incl = mine;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += v;
             }
+            __syncthreads();  // s_wcnt is no longer read
+            if (lane == 63) s_wcnt[wave] = incl;
+            __syncthreads();
+            int before = incl - mine, total = 0;
+            for (int v = 0; v < nwaves; v++) {
+                if (v < wave) before += s_wcnt[v];
+                total += s_wcnt[v];
+            }
+            int rs = nstart + (before & 0xffff), re = nseg + (before >> 16);
+            for (uint32_t left = starts; left != 0; left &= left - 1, rs++)
+                if (rs < kAppendSegList) s_start[rs] = t0 - 1 + __builtin_ctz(left);
+            for (uint32_t left = ends; left != 0; left &= left - 1, re++)
+                if (re < kAppendSegList) s_end[re] = t0 + __builtin_ctz(left);
+            nstart += total & 0xffff;
+            nseg += total >> 16;
+            if (nseg >= kAppendSegList) break;
+        }
+        __syncthreads();  // the lists are complete
+        if (nseg >= kAppendSegList) {
+            nseg = kAppendSegList;
+            resume = s_end[kAppendSegList - 1];
         }
         // Apply the complete segments, in order, one wave per (KV head, K|V).
         for (int p = part * nwaves + wave; p < 2 * num_kv_heads; p += parts * nwaves) {
             const int h = p >> 1;
             const bool is_v = (p & 1) != 0;
-            float amax = 0.0f, cur_scale = 0.0f;
-            bool have = false;  // statistics of an earlier pass are re-read (written before the barrier)
-            for (int k = 0; k < nseg; k++)
-                append_int8_apply<D>(is_v ? v_src : k_src, in_bf16, tok_stride, slot_at, s_start[k], s_end[k], blk,
-                                     is_v ? v_cache : k_cache, is_v ? v_scale : k_scale, is_v ? v_absmax : k_absmax,
-                                     h, num_kv_heads, is_v, amax, cur_scale, have);
+            append_int8_segments<D>(is_v ? v_src : k_src, in_bf16, tok_stride, slot_at, s_start, s_end, nseg, blk,
+                                    is_v ? v_cache : k_cache, is_v ? v_scale : k_scale, is_v ? v_absmax : k_absmax, h,
+                                    num_kv_heads, is_v, s_lut[wave]);
         }
         if (resume >= n_tok) break;
         __syncthreads();  // this pass's statistics and codes are visible to the next pass's waves

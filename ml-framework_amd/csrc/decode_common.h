@@ -599,7 +599,6 @@ constexpr int kMaxDecodeWorkers = 4096;   // workers (waves) of one MFMA decode 
 // one runs ahead and finishes first) but the chip's bandwidth stays in use either way; one 8-wave
 // workgroup per CU instead of two 4-wave ones measured slower.
 __host__ __device__ constexpr int decode_waves(int) { return 4; }
-int device_cus();
 // bf16 / int8 caches; num_seqs < kMaxPersistentSeqs. Launches the resident workgroups, each of
 // decode_waves(D) independent workers, with no more than kMaxDecodeWorkers and max_units workers
 // in all; records the worker count in a.split_grid (the merge kernel needs it).

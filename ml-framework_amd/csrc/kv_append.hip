@@ -6,6 +6,7 @@
 // PagedAttentionLayer.cs:315, with V transposed per tile): K tile [16 tokens][head_dim], V tile
 // [head_dim][16 tokens], one tile per (block, KV head). The append kernels are HBM-bound scatters;
 // the int8 one also owns the per-(block, KV head) scale and running absmax.
+#include <algorithm>
 #include <string>
 #include <type_traits>
 
@@ -266,38 +267,54 @@ __global__ __launch_bounds__(pa::kAppendMaxThreads) void append_int8_kernel(
                              v_absmax, num_kv_heads, capacity);
 }
 
-// int8 caches with 16-byte aligned operands: gridDim.y workgroups of up to kRunWaves waves per W
+// int8 caches with 16-byte aligned operands: gridDim.y workgroups of up to kRunWaves waves per kRunWindow
 // consecutive tokens of the call, a wave per (KV head, K|V). A token that starts a run of consecutive
 // slots of one block, when no other token of the call lands in that block (a prompt chunk's blocks, a
-// decode's tokens), has the run appended from registers (append_int8_run); a block whose tokens come in
-// any other way is left to append_int8_block, its (KV head, K|V) pairs shared by the workgroups. One
-// pass over the call's slots looks for other tokens of all the blocks that start here.
+// decode's tokens), has the run appended from registers (append_int8_run; one token: append_int8_apply); a
+// block whose tokens come in any other way is left to append_int8_block, its (KV head, K|V) pairs shared by
+// the workgroups. One pass over the call's slots looks for other tokens of all the blocks that start here.
 //
-// Latency-bound: slots, the look for other tokens and the run are three dependent round trips.
-// append_int8_block alone, a workgroup a token, takes a block's tokens one by one: 2048 tokens of 8 KV
-// heads of 128 in four chunks 64 us against 14.2 here, 16000 tokens 2270 against 79. W = 16 for calls
-// past kRunTokens: with a workgroup a token, 15 of 16 of a prompt's only read its slots, and a CU holds
-// few enough that they queue (28 us). The runs of a window, one for a prompt but up to 16 for scattered
-// tokens, are dealt to kRunShares workgroups (1000 decode tokens 32 us, as before, against 50 with
-// one). W = 1 below, where every token may be a run of its own (128 decode tokens 8.7 -> 6.7 us).
+// Latency-bound: the slots, then the run's values and its tile, are two dependent round trips. Against
+// append_int8_block alone, a workgroup a token (whose tokens of a block were applied segment by segment), us
+// of 8 KV heads of 128, bf16: prompt chunks of 4 x 512 210 -> 9.5, of 512 43 -> 7.4, 256 / 1000 decode tokens
+// 9.8 / 31.5 -> 8.9 / 24; 16 prompts of 64 tokens interleaved token by token 64 -> 55; 512 / 1024 tokens in random
+// order 58 / 61 -> 48 / 58 (2048: 64 -> 85, the look over the slots repeated by every workgroup).
+//
+// A window holds one start for a prompt and up to 16 for scattered tokens, which are dealt to gridDim.z
+// workgroups: as many as the chip holds, at least 4 (idle ones cost a prompt little: 4 x 512 tokens 9.5 us with 4
+// or 8, 11 with 16; 256 decode tokens take 12.7 with 4 and 8.9 with 12). With many KV heads a wave takes several pairs:
+// 2048 / n_tok workgroups a window, at least 4 (32 KV heads of 128: 256 decode tokens 15.5 us, with 16 workgroups 24;
+// prompts of 512 14.6 against 10).
 constexpr int kRunWaves = 4;
-constexpr int kRunTokens = 256;
-constexpr int kRunShares = 4;
-template <int D, bool IN_BF16, int W>
-__global__ __launch_bounds__(64 * kRunWaves) void append_int8_run_kernel(
+constexpr int kRunWindow = 16;
+constexpr int kRunPairs = 2048;
+template <int D, bool IN_BF16>
+__global__ __launch_bounds__(64 * kRunWaves, D > 128 ? 2 : D > 64 ? 3 : 4) void append_int8_run_kernel(
     const void* __restrict__ k_new, const void* __restrict__ v_new, const int64_t* __restrict__ slot_mapping,
     int32_t n_tok, int8_t* __restrict__ k_cache, int8_t* __restrict__ v_cache, float* __restrict__ k_scale,
     float* __restrict__ v_scale, float* __restrict__ k_absmax, float* __restrict__ v_absmax, int32_t num_kv_heads,
     int64_t capacity, int64_t tok_stride) {
-    __shared__ int s_blk[W], s_len[W], s_other;
+    constexpr int W = kRunWindow;
+    __shared__ int s_blk[W], s_len[W], s_other, s_before[W], s_segs[W];
     __shared__ __align__(16) int8_t s_stage[kRunWaves][pa::kBlockSize * D];
-    const int i0 = blockIdx.x * W;
+    // A window's workgroups on different XCDs (workgroups are dispatched to the 8 of them in turn).
+    const int i0 = static_cast<int>((blockIdx.x + blockIdx.y + gridDim.y * blockIdx.z) % gridDim.x) * W;
     const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // Lane l: token i0 - 1 + l's block (-1: none, skipped) and row, and whether it starts a segment of its block.
     const int64_t u = static_cast<int64_t>(i0) - 1 + lane;
     const int64_t sl = u >= 0 && u < n_tok ? slot_mapping[u] : -1;
     const int blk = sl >= 0 && sl < capacity ? static_cast<int>(sl >> 4) : -1, row = static_cast<int>(sl & 15);
+    // The first of the slots that the look for other tokens reads, in the same round trip.
+    int64_t o[pa::kAppendCoarse];
+    auto load_slots = [&](int t0) {
+#pragma unroll
+        for (int k = 0; k < pa::kAppendCoarse; k++) {
+            const int t = t0 + k * nthreads + tid;
+            o[k] = t < n_tok ? slot_mapping[t] : -1;
+        }
+    };
+    load_slots(0);
     const int prev = __shfl_up(blk, 1, 64);
     const uint64_t starts = __ballot(lane >= 1 && lane <= W && blk >= 0 && prev != blk);
     // The starts of a window are dealt to gridDim.z workgroups.
@@ -316,19 +333,17 @@ __global__ __launch_bounds__(64 * kRunWaves) void append_int8_run_kernel(
         if (tid == 0) {
             s_blk[l - 1] = b;
             s_len[l - 1] = __builtin_ctzll(~run);  // at most 16: the run stays in its block
+            s_before[l - 1] = 0;
+            s_segs[l - 1] = 1;
         }
     }
     if (tid == 0) s_other = 0;
     __syncthreads();
-    // Bit w of s_other: another token of the call lands in the block that starts at token i0 + w. Slots whose
-    // block's low six bits no such block has are passed over at once.
+    // Bit w of s_other: another token of the call lands in the block that starts at token i0 + w. s_segs[w]: how
+    // many segments of the block the call has; s_before[w]: how many before this one. Slots whose block's low
+    // six bits no such block has are passed over at once.
     for (int t0 = 0; t0 < n_tok; t0 += pa::kAppendCoarse * nthreads) {
-        int64_t o[pa::kAppendCoarse];
-#pragma unroll
-        for (int k = 0; k < pa::kAppendCoarse; k++) {
-            const int t = t0 + k * nthreads + tid;
-            o[k] = t < n_tok ? slot_mapping[t] : -1;
-        }
+        if (t0 > 0) load_slots(t0);
 #pragma unroll
         for (int k = 0; k < pa::kAppendCoarse; k++) {
             if (o[k] < 0 || o[k] >= capacity) continue;
@@ -336,7 +351,13 @@ __global__ __launch_bounds__(64 * kRunWaves) void append_int8_run_kernel(
             if (!((filter >> (b & 63)) & 1)) continue;
             for (uint64_t left = mine; left != 0; left &= left - 1) {
                 const int w = __builtin_ctzll(left) - 1;
-                if (b == s_blk[w] && (t < i0 + w || t >= i0 + w + s_len[w])) atomicOr(&s_other, 1 << w);
+                if (b != s_blk[w] || (t >= i0 + w && t < i0 + w + s_len[w])) continue;
+                atomicOr(&s_other, 1 << w);
+                const int64_t before = t > 0 ? slot_mapping[t - 1] : -1;
+                if (before < 0 || before >= capacity || static_cast<int>(before >> 4) != b) {
+                    atomicAdd(&s_segs[w], 1);
+                    if (t < i0 + w) atomicAdd(&s_before[w], 1);
+                }
             }
         }
     }
@@ -346,7 +367,10 @@ __global__ __launch_bounds__(64 * kRunWaves) void append_int8_run_kernel(
         const int l = __builtin_ctzll(left);
         const int i = i0 + l - 1;
         if ((others >> (l - 1)) & 1) {
-            pa::append_int8_block<D>(k_new, v_new, IN_BF16, tok_stride, [&](int t) { return slot_mapping[t]; }, i, n_tok,
+            // One of the block's segments, another one for other blocks, has the workgroup that owns it: were it
+            // the first, the call's first windows would own nearly all blocks of tokens out of order.
+            if (s_before[l - 1] != s_blk[l - 1] % s_segs[l - 1]) continue;
+            pa::append_int8_block<D, true>(k_new, v_new, IN_BF16, tok_stride, [&](int t) { return slot_mapping[t]; }, i, n_tok,
                                      k_cache, v_cache, k_scale, v_scale, k_absmax, v_absmax, num_kv_heads, capacity,
                                      static_cast<int32_t>(blockIdx.y), static_cast<int32_t>(gridDim.y));
             __syncthreads();  // its LDS is used again
@@ -357,6 +381,15 @@ __global__ __launch_bounds__(64 * kRunWaves) void append_int8_run_kernel(
         for (int p = static_cast<int>(blockIdx.y) * (nthreads >> 6) + wave; p < 2 * num_kv_heads;
              p += static_cast<int>(gridDim.y) * (nthreads >> 6)) {
             const bool v = (p & 1) != 0;
+            if (len == 1) {
+                float amax = 0.0f, scale = 0.0f;
+                bool have = false;
+                pa::append_int8_apply<D>(v ? v_new : k_new, IN_BF16, tok_stride,
+                                         [&](int) { return static_cast<int64_t>(b) * pa::kBlockSize + r0; }, i, i + 1, b,
+                                         v ? v_cache : k_cache, v ? v_scale : k_scale, v ? v_absmax : k_absmax, p >> 1,
+                                         num_kv_heads, v, amax, scale, have);
+                continue;
+            }
             pa::append_int8_run<D, IN_BF16>(v ? v_new : k_new, tok_stride, i, len, r0, b, v ? v_cache : k_cache,
                                             v ? v_scale : k_scale, v ? v_absmax : k_absmax, p >> 1, num_kv_heads, v,
                                             s_stage[wave]);
@@ -442,21 +475,20 @@ pa_status launch_kv_append(const char* f, hipStream_t s, const pa_config* cfg, c
         if (aligned) {
             const int tasks = 2 * cfg->num_kv_heads, waves = tasks < kRunWaves ? tasks : kRunWaves;
             const int ny = (tasks + waves - 1) / waves;
-            const bool wide = n_tok > kRunTokens;
-            const dim3 grid(wide ? (n_tok + 15) / 16 : n_tok, ny < 65535 ? ny : 65535, wide ? kRunShares : 1);
+            const int64_t windows = (static_cast<int64_t>(n_tok) + kRunWindow - 1) / kRunWindow;
+            // workgroups the chip holds, by the kernel's registers
+            const int64_t resident = (cfg->head_dim > 128 ? 2 : cfg->head_dim > 64 ? 3 : 4) * static_cast<int64_t>(device_cus());
+            const int y = std::min(ny, std::max(4, kRunPairs / n_tok));
+            const int z = static_cast<int>(std::min<int64_t>(std::min(kRunWindow, n_tok), std::max<int64_t>(4, resident / (windows * y))));
+            const dim3 grid(static_cast<unsigned>(windows), y, z);
             auto go = [&](auto kern) {
                 kern<<<grid, 64 * waves, 0, s>>>(k_new, v_new, slot_mapping, n_tok, kc, vc, k_scale, v_scale, k_absmax,
                                                  v_absmax, cfg->num_kv_heads, capacity, tok_stride);
             };
             switch (cfg->head_dim) {
-#define PA_APPEND_RUN(DD)                                                                                     \
-    if (wide) go(in_bf16 ? append_int8_run_kernel<DD, true, 16> : append_int8_run_kernel<DD, false, 16>);       \
-    else go(in_bf16 ? append_int8_run_kernel<DD, true, 1> : append_int8_run_kernel<DD, false, 1>);            \
-    break;
-                case 64: PA_APPEND_RUN(64)
-                case 128: PA_APPEND_RUN(128)
-                default: PA_APPEND_RUN(256)
-#undef PA_APPEND_RUN
+                case 64: go(in_bf16 ? append_int8_run_kernel<64, true> : append_int8_run_kernel<64, false>); break;
+                case 128: go(in_bf16 ? append_int8_run_kernel<128, true> : append_int8_run_kernel<128, false>); break;
+                default: go(in_bf16 ? append_int8_run_kernel<256, true> : append_int8_run_kernel<256, false>); break;
             }
             PA_HIP_CHECK(hipGetLastError());
             return clear_error();

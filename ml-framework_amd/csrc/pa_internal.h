@@ -148,12 +148,13 @@ __device__ __forceinline__ float wave_sum(float v) {
 __device__ __forceinline__ int8_t quantize_symmetric(float v, float scale) {
 #pragma clang fp contract(off)
     float scaled = v / scale;  // IEEE division (hipcc default: correctly rounded fp32 divide)
-    if (scaled != scaled) return 0;  // NaN (value NaN, 0/0) -> 0
     float a = floorf(fabsf(scaled) + 0.5f);
-    float r = copysignf(a, scaled);
-    if (r >= 127.0f) return 127;
-    if (r <= -128.0f) return -128;
-    return static_cast<int8_t>(static_cast<int>(r));
+    float r = fminf(fmaxf(copysignf(a, scaled), -128.0f), 127.0f);
+    // selected, not branched to: the callers quantise values by the dozen
+    return static_cast<int8_t>(scaled != scaled ? 0 : static_cast<int>(r));  // NaN (value NaN, 0/0) -> 0
 }
+
+// CUs of the current device (paged_decode.hip).
+int device_cus();
 
 }  // namespace pa

@@ -347,6 +347,52 @@ def test_append_int8_out_of_order_bit_exact(stream, D, q_dtype):
     step(slots, [0.25, 1.0, 8.0])
 
 
+@pytest.mark.parametrize("D,q_dtype,hkv,shift", [(128, 0, 3, 0), (64, 1, 1, 0), (256, 1, 2, 0), (128, 1, 10, 0),
+                                                 (128, 0, 3, 1), (64, 1, 8, 1), (256, 0, 1, 1)])
+def test_append_int8_interleaved_bit_exact(stream, D, q_dtype, hkv, shift):
+    """Blocks whose tokens are many segments of the call, from short calls to several windows of tokens: prompts
+    interleaved token by token, a random order, a reversed one, rows written again and again in one segment of
+    more than 64 tokens and in many; new K/V 16-byte aligned (shift 0) or one element off it."""
+    rng = np.random.default_rng(290 + D + hkv)
+    nb = 40
+    cfg = pa.make_config(num_q_heads=hkv, num_kv_heads=hkv, head_dim=D, kv_dtype=2, q_dtype=q_dtype,
+                         num_blocks=nb)
+    host = dict(kc=np.zeros((nb, hkv, 16, D), np.int8), vc=np.zeros((nb, hkv, 16, D), np.int8),
+                ks=np.zeros((nb, hkv), np.float32), vs=np.zeros((nb, hkv), np.float32),
+                ka=np.zeros((nb, hkv), np.float32), va=np.zeros((nb, hkv), np.float32))
+    dev = {n: to_gpu(a) for n, a in host.items()}
+
+    def step(slots, mults=(1.0,)):
+        slots = np.asarray(slots, np.int64)
+        mult = rng.choice(mults, size=(len(slots), 1, 1)).astype(np.float32)
+        k = (rng.standard_normal((len(slots), hkv, D), dtype=np.float32) * mult).astype(np.float32)
+        v = (rng.standard_normal((len(slots), hkv, D), dtype=np.float32) * mult[::-1]).astype(np.float32)
+        k[len(slots) // 3, 0, 1] = np.nan
+        if q_dtype == 1:
+            k, v = orc.bf16_from_f32(k), orc.bf16_from_f32(v)
+        orc.kv_append(cfg, k, v, slots, host["kc"], host["vc"], host["ks"], host["vs"], host["ka"], host["va"])
+        gpu = [to_gpu(np.concatenate([np.zeros(shift, a.dtype), a.reshape(-1)]))[shift:] for a in (k, v)]
+        pa.kv_append(stream, cfg, *gpu, to_gpu(slots), len(slots), dev["kc"], dev["vc"], dev["ks"], dev["vs"], dev["ka"],
+                     dev["va"])
+        _sync()
+        for n, a in host.items():
+            np.testing.assert_array_equal(to_np(dev[n]), a, err_msg=n)
+
+    def prompts(blocks, start, n):  # [token][prompt]: n tokens from row `start` of each row of blocks
+        pos = start + np.arange(n)
+        return (blocks[:, pos // 16] * 16 + pos % 16).T
+
+    perm = rng.permutation(nb)
+    step(prompts(perm[:4].reshape(2, 2), 0, 9).reshape(-1))                       # 18 tokens
+    step(prompts(perm[:4].reshape(2, 2), 9, 20).reshape(-1), (0.5, 4.0))
+    step(prompts(perm[4:].reshape(6, 6), 3, 70).reshape(-1), (0.5, 2.0))           # 420 tokens, six at a time
+    step(rng.permutation(prompts(perm[:36].reshape(9, 4), 0, 60).reshape(-1)), (0.25, 1.0, 8.0))
+    step(np.concatenate([np.arange(16)[::-1] + 16 * perm[1], np.arange(7, 12)[::-1] + 16 * perm[2]]))
+    again = rng.integers(0, 16, 100) + 16 * perm[5]                                # one segment
+    step(np.concatenate([again, [16 * perm[6] + 3], rng.integers(1, 16, 70) + 16 * perm[5], [-1], again[:3]]), (0.5, 3.0))
+    step(rng.integers(0, 16, 300) + 16 * perm[rng.integers(7, 9, 300)], (0.5, 3.0))  # more segments than a list
+
+
 @pytest.mark.parametrize("old_scale,new_amax", [(0.5, 127.0), (0.0078125, 3.0), (0.2618793547153473, 95.5709228515625),
                                                (1.7, 1e4)])
 def test_append_int8_requantisation_all_codes(stream, old_scale, new_amax):
