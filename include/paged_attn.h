@@ -349,9 +349,9 @@ pa_status pa_paged_decode_prefix(pa_stream* stream, const pa_config* cfg, float*
  *   max_chunk_len: host-side upper bound of the chunk lengths.
  * Range: every finite cache value is accepted. The P.V product runs on fp16 operands; int8
  * caches fold log2 of each block's V scale into the softmax exponent, so P times the scale stays
- * within fp16 for any scale; bf16 caches whose V tiles hold a magnitude above 65504 (fp16's
- * largest) are detected as the tiles are converted, and the query tiles that read them are
- * computed again in fp32 (a slower path, taken only for such inputs). */
+ * within fp16 for any scale; query tiles that read a V magnitude above 65504 (fp16's largest)
+ * from a bf16 cache are detected and computed again in fp32 (a slower path, taken only for such
+ * inputs). Queries and keys that are not finite give outputs that are not, at the usual speed. */
 pa_status pa_chunked_prefill(pa_stream* stream, const pa_config* cfg, float* out, const void* q,
                              const int32_t* q_start_loc, const int32_t* prefix_lens,
                              const void* k_cache, const void* v_cache,

@@ -214,6 +214,35 @@ __device__ void prefill_exact_unit(const PrefillArgs& a, const int32_t* table, i
     }
 }
 
+// Whether the first nkb blocks of a sequence hold V values that an fp16 P.V product cannot take: magnitudes from
+// 65536 (the least bf16 above fp16's largest) to infinity, or a NaN at a key `lim` or later, which not
+// every query of the unit sees (0 times it is NaN for the others; where all see it, NaN is the result). One
+// wave, once for a unit whose output is not finite.
+template <int D>
+__device__ bool prefill_v_beyond_fp16(const PrefillArgs& a, const int32_t* table, int kvh, int nkb, int lim) {
+    const int lane = threadIdx.x & 63;
+    for (int b = 0; b < nkb; b++) {
+        const int id = table[b];
+        if (id < 0 || id >= a.num_blocks) continue;
+        const uint4* tile = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.v_cache) +
+                                                           (static_cast<int64_t>(id) * a.num_kv_heads + kvh) * 16 * D);
+        bool hit = false;
+#pragma unroll
+        for (int j = 0; j < D / 32; j++) {
+            const int c = lane + 64 * j;  // dim c / 2, tokens 8 (c % 2) .. + 7
+            const uint4 x = tile[c];
+            const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t m = (w[e >> 1] >> (16 * (e & 1))) & 0x7fffu;
+                hit = hit || (m >= 0x4780u && (m <= 0x7f80u || 16 * b + 8 * (c & 1) + e >= lim));
+            }
+        }
+        if (__any(hit)) return true;
+    }
+    return false;
+}
+
 // The units of round u0 of this workgroup that this wave computes (the kernel's decomposition,
 // rederived from the arguments so that nothing stays live across the stream for this rare path),
 // through prefill_exact_unit.
@@ -1187,17 +1216,22 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>(
         for (int i = 0; i < 4; i++) {
             const int qi = 4 * q4 + i;
             if (qi < nq[k]) {
-                const float inv = 1.0f / __shfl(l_tot, qi, 64);
+                const float l = __shfl(l_tot, qi, 64);
+                const float inv = 1.0f / l;
+                const bool sum_ok = (__float_as_uint(l) & 0x7f800000u) != 0x7f800000u;
                 float* op = a.out + (static_cast<int64_t>(q0 + i0[k] + qi) * Hq + head[k]) * D;
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
-                    if constexpr (ELT == 2) bad = bad || (__float_as_uint(acc[k][t][i]) & 0x7f800000u) == 0x7f800000u;
+                    if constexpr (ELT == 2)
+                        bad = bad || (sum_ok && (__float_as_uint(acc[k][t][i]) & 0x7f800000u) == 0x7f800000u);
                     op[16 * t + n] = acc[k][t][i] * inv;
                 }
             }
         }
         if constexpr (ELT == 2) {
-            if (__any(bad))
+            // An output that is not finite though its row's sum is: V beyond fp16, or V itself not finite. (A sum that
+            // is not has its cause in Q or K, which nothing computed again would change.)
+            if (__any(bad) && prefill_v_beyond_fp16<D>(a, table, kvh, nkb, causal ? min(T, P + i0[k] + 1) : T))
                 prefill_exact_unit<D, QF32>(a, table, kvh, head[k], q0 + i0[k], nq[k], P + i0[k], T, causal);
         }
     }

@@ -201,6 +201,67 @@ def test_prefill_values_beyond_fp16_range(stream, flags, kv_dtype, q_dtype, Hq, 
     check_close(got / f, ref / f, **tol_for(kv_dtype), what=f"large V kv={kv_dtype} D={D} flags={flags} x{f}")
 
 
+def _timed_prefill(stream, edit, repeat=3):
+    """Shortest time of a 64-query chunk behind 2000 tokens (waves sharing the keys), inputs edited, and its output."""
+    import torch
+
+    w = wl.make_small(390, num_seqs=1, lens=[2064], Hq=4, Hkv=1, D=128, kv_dtype=1, q_dtype=1)
+    inp = wl.numpy_inputs(w, 391)
+    q = orc.bf16_from_f32(np.random.default_rng(392).standard_normal((64, 4, 128)).astype(np.float32))
+    blk = w.block_tables[0]
+    edit(q, inp["k_cache"].reshape(w.num_blocks, 1, 16, 128), inp["v_cache"].reshape(w.num_blocks, 1, 128, 16), blk)
+    out = empty_gpu((64, 4, 128), np.float32)
+    args = (to_gpu(q), to_gpu(np.array([0, 64], np.int32)), to_gpu(np.array([2000], np.int32)), to_gpu(inp["k_cache"]),
+            to_gpu(inp["v_cache"]), None, None, to_gpu(w.block_tables), 1, w.max_blocks, 64)
+    best = 1e9
+    for _ in range(repeat + 1):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        pa.chunked_prefill(stream, config_for(w), out, *args)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best, to_np(out)
+
+
+def test_prefill_nan_inputs_at_the_usual_speed(stream):
+    """A NaN in a query, a key or a value every query sees makes the outputs that depend on it NaN, without the
+    one-key-at-a-time path kept for V magnitudes that fp16 cannot hold (hundreds of times the usual time)."""
+    NAN, BIG = 0x7fc0, 0x4800  # bf16: NaN, 131072
+
+    def clean(q, k, v, blk):
+        pass
+
+    def nan_q(q, k, v, blk):
+        q[7, 1, 3] = NAN
+
+    def nan_k(q, k, v, blk):
+        k[blk[5], 0, 4, 9] = NAN
+
+    def nan_v(q, k, v, blk):
+        v[blk[5], 0, 11, 4] = NAN
+
+    def big_v_nan_q(q, k, v, blk):
+        q[7, 1, 3] = NAN
+        v[blk[100], 0, 11, 4] = BIG
+
+    usual, ref = _timed_prefill(stream, clean)
+    assert np.isfinite(ref).all()
+    t, out = _timed_prefill(stream, nan_q)
+    assert t < 20 * usual and np.isnan(out[7, 1]).all()
+    np.testing.assert_array_equal(np.isnan(out).sum(), 128)
+    t, out = _timed_prefill(stream, nan_k)
+    assert t < 20 * usual and np.isnan(out).all()
+    t, out = _timed_prefill(stream, nan_v)
+    assert t < 20 * usual and np.isnan(out[:, :, 11]).all() and np.isnan(out).sum() == 64 * 4
+    _, out = _timed_prefill(stream, big_v_nan_q)
+    assert np.isnan(out[7, 1]).all() and np.isnan(out).sum() == 128
+    keep = np.ones_like(out, bool)
+    keep[7, 1], keep[:, :, 11] = False, False
+    check_close(out[keep], ref[keep], **tol_for(1), what="dims without the large value")
+    assert (out[:, :, 11] > ref[:, :, 11])[np.isfinite(out[:, :, 11])].all()
+
+
 @pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D,prefix,chunk", [
     (1, 1, 8, 2, 128, [223, 0, 255, 16], [33, 1, 16, 250]),   # heads of a tile; queries some waves have no key for
     (1, 0, 6, 2, 128, [300, 7], [17, 48]),                    # G = 3: units of a workgroup span two tiles
