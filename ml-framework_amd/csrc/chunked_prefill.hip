@@ -773,19 +773,23 @@ __global__ __launch_bounds__(kPrefillThreads, D > 128 ? 1 : (D > 64 && QF32 ? 2 
 // The kernel above gives a workgroup's waves one stream of keys and different units; a call whose
 // workgroups do not fill the chip (one 512-token chunk of a Llama-shaped layer is 128 of them) then
 // waits on the serial chain over the keys, about 0.92 us per pair of blocks for a workgroup alone
-// on its CU. Here a workgroup takes NU = 4 units (2 for head_dim 256) and its 8 waves split the
-// keys: wave w streams pairs w, w + 8, .. of the block list through an LDS slot of its own and
-// computes all four units on them, and the waves' (max, sum, O) are added up through LDS at the
-// end. No wave waits for another in the stream (eight waves stepping together behind a barrier
-// measured 59 us where this one takes 46), a K operand read from LDS feeds four units and a V
-// operand is converted to fp16 once for four. One slot a wave is enough: the next pair's K loads
-// go out when the QK products have read the slot's K, its V loads after the PV products, and the
-// SIMD's other wave runs while they land.
+// on its CU. Here a workgroup takes NU units, 1 or 2 where that is enough for one workgroup a CU, else 4
+// (2 for head_dim 256), and its waves (8, or 4 where two a SIMD do not fit) split the keys: wave w streams
+// pairs w, w + 8, .. of the block list through an LDS slot of its own and computes all the units on
+// them, and the waves' (max, sum, O) are added up through LDS at the end. No wave waits for another in
+// the stream (eight waves stepping together behind a barrier measured 59 us where this one takes 46), a
+// K operand read from LDS feeds NU units and a V operand is converted to fp16 once for them. One slot a
+// wave is enough: the next pair's K loads go out when the QK products have read the slot's K, its V
+// loads after the PV products, and the SIMD's other wave runs while they land.
 //
-// What bounds it: VALU issue (softmax, V conversion) and MFMA, which two waves a SIMD overlap only
-// in part: about 2300 clocks per pair and wave against 1400 of VALU and 1020 of MFMA. A 512-token
-// chunk on 3333 tokens, Llama shape (32 / 8 heads of 128, bf16): 109.5 -> 46 us (660 TFLOP/s); 20
-// tokens on 8000: 220 -> 71; int8 cache, 512 on 2000: 109 -> 44.
+// What bounds it: with NU = 4, VALU issue (softmax, V conversion) and MFMA, which two waves a SIMD
+// overlap only in part: about 2300 clocks per pair and wave against 1400 of VALU and 1020 of MFMA. A
+// 512-token chunk on 3333 tokens, Llama shape (32 / 8 heads of 128, bf16): 109.5 -> 46 us (660
+// TFLOP/s); int8 cache, 512 on 2000: 109 -> 43. (The instances of head_dim 128 and bf16 queries spill 13
+// registers, 41 over int8 caches, whose reloads the compiler waits for in the counter that the loop's own
+// loads share: in part they undo the prefetch.) With few units, the loads through LDS, and for short
+// contexts the launch and its round trips: 20 tokens on 8000 217 -> 39 us (71 with NU = 4), 203 tokens
+// 11.6 -> 9.8 (13.2).
 
 // LDS-direct loads of one tile of SEG KiB, 16 bytes a lane: segment j at immediate offset 1024 j,
 // which advances both the memory and the LDS address; off0 / off1 are the lane's offset within an
@@ -828,20 +832,23 @@ __device__ __forceinline__ void lds_load_tile(u32x4_t r, uint32_t off0, uint32_t
     }
 }
 
-// Units of a workgroup (each wave holds the accumulators of all of them) and its waves: two a SIMD,
-// one where 512 registers are needed (head_dim 256, or the low parts of fp32 queries).
+// Units of a workgroup, at most (each wave holds the accumulators of all of them), and its waves: two a
+// SIMD, one where 512 registers are needed (head_dim 256, or the low parts of fp32 queries).
 __host__ __device__ constexpr int wave_units(int d) { return d > 128 ? 2 : 4; }
-template <int D, bool QF32> __host__ __device__ constexpr int wave_waves() { return D > 128 || (D > 64 && QF32) ? 4 : 8; }
+template <int D, bool QF32, int NU> __host__ __device__ constexpr int wave_waves() {
+    return D > 128 || (D > 64 && QF32 && NU == wave_units(D)) ? 4 : 8;
+}
 
 // LDS of the kernel, one dynamic array: the compiler, which would see that only one workgroup fits
 // a CU, otherwise allots 512 registers a wave and moves the accumulators between the two halves of
 // the register file on every step.
-template <int D, int KV, bool QF32> struct WaveLds {
+template <int D, int KV, bool QF32, int NU> struct WaveLds {
     using TL = PrefillTile<D, MfmaRaw<KV>::kElt>;
-    static constexpr int WAVES = wave_waves<D, QF32>();
-    static constexpr int UNITS = wave_units(D);
+    static constexpr int WAVES = wave_waves<D, QF32, NU>();
+    static constexpr int UNITS = NU;
+    static constexpr bool FEW = NU < wave_units(D);              // every wave's states fit at once
     static constexpr int NST = D / 16;                           // 16-byte words per lane of a unit's state
-    static constexpr int STATES = (WAVES > 4 ? 4 : 3) * UNITS;   // states exchanged at a time
+    static constexpr int STATES = (FEW ? WAVES : WAVES > 4 ? 4 : 3) * UNITS;  // states exchanged at a time
     static constexpr int TILES = WAVES * TL::SLOT > STATES * NST * 64 ? WAVES * TL::SLOT : STATES * NST * 64;
     static constexpr int Q = UNITS * (D / 32) * 64;
     static constexpr int KCH = KV == PA_DTYPE_INT8 ? 512 : 1024;  // block ids (and int8 scales) at a time
@@ -851,23 +858,23 @@ template <int D, int KV, bool QF32> struct WaveLds {
         uint4 q[Q];              // Q operands
         float2 ml[STATES * 64];  // the states' (max, row sum)
     };
+    int beyond;  // units with an output that is not finite
     int ids[KCH + PAD];
     float ksc[KV == PA_DTYPE_INT8 ? KCH + PAD : 1], vlg[KV == PA_DTYPE_INT8 ? KCH + PAD : 1],
         vrc[KV == PA_DTYPE_INT8 ? KCH + PAD : 1];
 };
 
-template <int D, int KV, bool QF32>
-__global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>() / 4)) void chunked_prefill_wave_kernel(const PrefillArgs a) {
+template <int D, int KV, bool QF32, int NU>
+__global__ __launch_bounds__((64 * wave_waves<D, QF32, NU>()), (wave_waves<D, QF32, NU>() / 4)) void chunked_prefill_wave_kernel(const PrefillArgs a) {
     using Raw = MfmaRaw<KV>;
     constexpr int ELT = Raw::kElt;
     constexpr int NSLAB = D / 32;
     constexpr int NT = D / 16;
     constexpr int TILE = 16 * D;
-    constexpr int NU = wave_units(D);
     using KR = typename Raw::K;
     using TL = PrefillTile<D, ELT>;
     constexpr int SEG = TL::SPT;             // KiB of a tile
-    using L = WaveLds<D, KV, QF32>;
+    using L = WaveLds<D, KV, QF32, NU>;
     constexpr int WAVES = L::WAVES, NST = L::NST, KCH = L::KCH, kPad = L::PAD;
     extern __shared__ __align__(16) char wave_lds[];
     L& sh = *reinterpret_cast<L*>(wave_lds);
@@ -1009,7 +1016,7 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>(
             }
         }
         __syncthreads();
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the loop counts its own loads only
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the loop's waits count its own loads (and reloads, if any)
         // ids of steps st .. st + 31 (st a multiple of 32) of this wave
         auto refill = [&](int st) {
             const int j = 2 * wave + 2 * WAVES * (st + (lane >> 1)) + (lane & 1);
@@ -1155,7 +1162,81 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>(
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS-direct write outlives the chunk
     }
-    __syncthreads();  // the rings are no longer read: they take the units' states
+    const int busy = min(WAVES, (nkb + 1) / 2);  // waves past the last pair of blocks have no state to leave
+    const int lim0 = P + 1;  // unit k: every query of it sees the keys below lim0 + i0[k]
+    if constexpr (L::FEW) {
+        // Every wave leaves its states; 16-dim piece i = NT k + t of the units is added up and stored by wave
+        // i % WAVES.
+        if (tid == 0) sh.beyond = 0;
+        __syncthreads();  // the slots are no longer read: they take the states
+        if (wave < busy) {
+#pragma unroll
+            for (int k = 0; k < NU; k++) {
+                uint4* st = s_tile + (wave * NU + k) * 64 * NST + lane;
+#pragma unroll
+                for (int t = 0; t < NT; t++) st[64 * t] = __builtin_bit_cast(uint4, acc[k][t]);
+                s_ml[(wave * NU + k) * 64 + lane] = make_float2(m_run[k], l_run[k]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NU; k++) {
+            float2 ml[WAVES];
+            float mt = -__FLT_MAX__, l = 0.0f;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                ml[w] = w < busy ? s_ml[(w * NU + k) * 64 + lane] : make_float2(-__FLT_MAX__, 0.0f);
+                mt = fmaxf(mt, ml[w].x);
+            }
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                ml[w].x = __builtin_amdgcn_exp2f(ml[w].x - mt);
+                l += ml[w].y * ml[w].x;
+            }
+            const float l_tot = rows_sum(l);  // query n's, in every lane of column n
+            float lq[4], inv[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                lq[e] = __shfl(l_tot, 4 * q4 + e, 64);
+                inv[e] = 1.0f / lq[e];
+            }
+            bool bad = false;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                if ((k * NT + t) % WAVES != wave) continue;
+                float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int w = 0; w < WAVES; w++) {
+                    if (w >= busy) break;
+                    const f32x4_t x = __builtin_bit_cast(f32x4_t, s_tile[((w * NU + k) * NST + t) * 64 + lane]);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[e] += x[e] * __shfl(ml[w].x, 4 * q4 + e, 64);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (4 * q4 + e >= nq[k]) continue;
+                    if constexpr (ELT == 2)
+                        bad = bad || ((__float_as_uint(lq[e]) & 0x7f800000u) != 0x7f800000u &&
+                                      (__float_as_uint(o[e]) & 0x7f800000u) == 0x7f800000u);
+                    a.out[(static_cast<int64_t>(q0 + i0[k] + 4 * q4 + e) * Hq + head[k]) * D + 16 * t + n] = o[e] * inv[e];
+                }
+            }
+            if constexpr (ELT == 2) {
+                if (__any(bad) && lane == 0) atomicOr(&sh.beyond, 1 << k);
+            }
+        }
+        if constexpr (ELT == 2) {
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the stores precede those of the fallback
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < NU; k++)  // see the other ending
+                if (k == wave && (sh.beyond >> k & 1) &&
+                    prefill_v_beyond_fp16<D>(a, table, kvh, nkb, causal ? min(T, lim0 + i0[k]) : T))
+                    prefill_exact_unit<D, QF32>(a, table, kvh, head[k], q0 + i0[k], nq[k], P + i0[k], T, causal);
+        }
+        return;
+    }
+    __syncthreads();  // the slots are no longer read: they take the units' states
 
     // The waves' states are added up through LDS, the sums brought to the larger maximum. State i of
     // unit k: 16-byte word t of a lane at 64 t + lane.
@@ -1185,9 +1266,7 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>(
             for (int e = 0; e < 4; e++) acc[k][t][e] = acc[k][t][e] * r0[e] + x[e] * r1[e];
         }
     };
-    // Waves 4 .. 7 leave theirs to waves 0 .. 3, which then each end one unit. Waves past the last
-    // pair of blocks have none to leave.
-    const int busy = min(WAVES, (nkb + 1) / 2);
+    // Waves 4 .. 7 leave theirs to waves 0 .. 3, which then each end one unit.
     if (WAVES > 4 && busy > 4) {
         if (wave >= 4 && wave < busy) {
 #pragma unroll
@@ -1231,22 +1310,30 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32>()), (wave_waves<D, QF32>(
         if constexpr (ELT == 2) {
             // An output that is not finite though its row's sum is: V beyond fp16, or V itself not finite. (A sum that
             // is not has its cause in Q or K, which nothing computed again would change.)
-            if (__any(bad) && prefill_v_beyond_fp16<D>(a, table, kvh, nkb, causal ? min(T, P + i0[k] + 1) : T))
+            if (__any(bad) && prefill_v_beyond_fp16<D>(a, table, kvh, nkb, causal ? min(T, lim0 + i0[k]) : T))
                 prefill_exact_unit<D, QF32>(a, table, kvh, head[k], q0 + i0[k], nq[k], P + i0[k], T, causal);
         }
     }
 }
 
-template <int D, int KV, bool QF32>
-void launch(const PrefillArgs& a, bool wave, dim3 grid, hipStream_t s) {
-    using L = WaveLds<D, KV, QF32>;
+template <int D, int KV, bool QF32, int NU>
+void launch_wave(const PrefillArgs& a, dim3 grid, hipStream_t s) {
+    using L = WaveLds<D, KV, QF32, NU>;
     static_assert(sizeof(L) <= 160 << 10, "the LDS of a CU");
-    if (wave) chunked_prefill_wave_kernel<D, KV, QF32><<<grid, 64 * L::WAVES, sizeof(L), s>>>(a);
-    else chunked_prefill_kernel<D, KV, QF32><<<grid, kPrefillThreads, 0, s>>>(a);
+    chunked_prefill_wave_kernel<D, KV, QF32, NU><<<grid, 64 * L::WAVES, sizeof(L), s>>>(a);
+}
+
+// wave: units of a workgroup of the wave-split kernel; 0: the other one.
+template <int D, int KV, bool QF32>
+void launch(const PrefillArgs& a, int wave, dim3 grid, hipStream_t s) {
+    if (wave == 0) chunked_prefill_kernel<D, KV, QF32><<<grid, kPrefillThreads, 0, s>>>(a);
+    else if (wave == 1) launch_wave<D, KV, QF32, 1>(a, grid, s);
+    else if (wave == 2) launch_wave<D, KV, QF32, 2>(a, grid, s);
+    else if constexpr (wave_units(D) > 2) launch_wave<D, KV, QF32, wave_units(D)>(a, grid, s);
 }
 
 template <int D>
-void launch_kv(const PrefillArgs& a, bool wave, int kv, bool qf32, dim3 grid, hipStream_t s) {
+void launch_kv(const PrefillArgs& a, int wave, int kv, bool qf32, dim3 grid, hipStream_t s) {
     if (kv == PA_DTYPE_BF16) {
         if (qf32) launch<D, PA_DTYPE_BF16, true>(a, wave, grid, s);
         else launch<D, PA_DTYPE_BF16, false>(a, wave, grid, s);
@@ -1306,15 +1393,27 @@ extern "C" pa_status pa_chunked_prefill(pa_stream* stream, const pa_config* cfg,
 
     const int64_t ng = static_cast<int64_t>(num_seqs) * cfg->num_kv_heads;
     const int64_t tiles = (static_cast<int64_t>(max_chunk_len) + 15) / 16;
-    // Calls whose workgroups the wave-split kernel runs in one generation (one a CU) go to it when
-    // there may be keys to split (256: 13.0 against 13.6 us without a prefix, 19.9 against 16.3 with 256
-    // tokens), calls of one and a half to two generations when the context may reach 1024 tokens
-    // (2 x 512 on 800 tokens 43.7 against 40.6 us; 1024 on 2000 88 against 64.5; three generations: 54
-    // against 59). The table's width bounds the context; the prefix lengths are on the device.
-    const int units = pa::wave_units(cfg->head_dim);
-    const int64_t wave_wgs = (tiles * a.group + units - 1) / units;
-    const int64_t cus = pa::device_cus(), w = ng * wave_wgs;
-    bool wave = (w <= cus && max_blocks_per_seq >= 16) || (2 * w > 3 * cus && w <= 2 * cus && max_blocks_per_seq >= 64);
+    // The wave-split kernel takes the calls that it runs in one generation of workgroups, one a CU, with the
+    // fewest units a workgroup. With less than its most units it is the faster one whatever the context (32 / 8
+    // heads of 128, bf16, us: 16 tokens 6.9 -> 5.8, on 700 24.8 -> 9.8; 203 tokens 11.6 -> 10.0, on 700 29.6 -> 14.5).
+    // With its most, from contexts of about 320 tokens on (8 x 64 tokens 9.1 -> 10.4, on 200 14.6 -> 15.7, on 700
+    // 28.6 -> 20.2; 2 x 256 13.8 -> 14.6, on 200 19.7 -> 17.0; one chunk of more than 256: always).
+    // Calls of one and a half to two generations go to it for one long chunk (1024 tokens 34.4 -> 31.8, on 2000 86
+    // -> 67), or where the context may reach 1536 tokens (2 x 512 on 200 28.2 -> 32.4, on 700 40.8 -> 41.5, on 2000 75
+    // -> 64); shorter chunks lose more than they gain (4 x 256 15.6 -> 25.8, on 2000 70 -> 63). head_dim 256: from
+    // 768 tokens on (8 x 128 17 -> 23, on 200 29 -> 33, on 700 54 -> 45, on 2000 123 -> 81).
+    // The prefix lengths are on the device: the table's width bounds the context, so a caller whose tables are wider
+    // than its contexts pays the differences above.
+    const int64_t cus = pa::device_cus();
+    const int most = pa::wave_units(cfg->head_dim);
+    int units = 1;
+    while (units < most && ng * ((tiles * a.group + units - 1) / units) > cus) units *= 2;
+    const int64_t wave_wgs = (tiles * a.group + units - 1) / units, w = ng * wave_wgs;
+    const bool two = cfg->head_dim > 128 ? max_blocks_per_seq >= 48
+                                         : max_chunk_len > 768 || (max_chunk_len >= 512 && max_blocks_per_seq >= 96);
+    const bool fits = w <= cus ? units < most || max_chunk_len > 256 || max_blocks_per_seq >= 20
+                               : 2 * w > 3 * cus && w <= 2 * cus && two;
+    const int wave = fits ? units : 0;
     a.qtiles_per_wg = a.group >= pa::kPrefillUnits ? 1 : pa::kPrefillUnits / a.group;
     const int64_t qgroups = wave ? wave_wgs : (tiles + a.qtiles_per_wg - 1) / a.qtiles_per_wg;
     a.num_qgroups = static_cast<int32_t>(qgroups);

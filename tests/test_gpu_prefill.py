@@ -271,9 +271,27 @@ def test_prefill_nan_inputs_at_the_usual_speed(stream):
     (2, 1, 16, 1, 64, [260, 9], [2, 31]),
     (1, 1, 8, 1, 256, [400, 0], [40, 16]),
     (2, 0, 2, 2, 256, [241, 270], [15, 1]),
+    (1, 1, 4, 4, 128, [5, 300, 77], [33, 20, 3]),             # 12 (sequence, KV head) groups: 8 and a remainder
+    (1, 0, 3, 1, 64, [0, 20, 7, 64, 3, 40, 1, 90, 15, 16, 200], [17] * 11),   # 11
+    # more than 512 units (256 for head_dim 256): the most units a workgroup takes, in one generation of them
+    (1, 1, 32, 8, 128, [223, 0, 255, 16], [33, 1, 128, 120]),
+    (1, 0, 24, 8, 128, [300, 7, 0], [17, 140, 130]),           # G = 3
+    (2, 0, 32, 8, 128, [400, 0, 33], [130, 16, 97]),
+    (2, 1, 32, 8, 128, [8180, 0], [30, 256]),                   # int8 scales past 512 blocks
+    (1, 1, 16, 16, 64, [500, 0, 31], [200, 130, 256]),          # G = 1: four tiles a workgroup
+    (1, 0, 32, 16, 64, [16370, 3], [18, 144]),                  # keys past 1024 blocks
+    (2, 1, 16, 1, 64, [260, 9, 0], [200, 180, 1]),
+    (2, 0, 64, 8, 64, [305, 0], [70, 100]),
+    (1, 1, 16, 2, 256, [400, 0], [40, 144]),
+    (1, 0, 16, 4, 256, [330, 9], [144, 80]),
+    (2, 1, 16, 4, 256, [241, 270], [130, 100]),
+    (2, 0, 16, 2, 256, [20, 350], [140, 1]),
+    # one and a half to two generations
+    (1, 1, 32, 8, 128, [0], [800]),
+    (2, 0, 16, 4, 256, [700, 0], [150, 410]),
 ])
 def test_prefill_keys_split_over_waves(stream, kv_dtype, q_dtype, Hq, Hkv, D, prefix, chunk):
-    """Few workgroups and tables of 16 blocks or more: the waves of a workgroup split its keys."""
+    """Calls of few workgroups, whose waves split its keys."""
     got, ref = run_prefill(stream, prefix=prefix, chunk=chunk, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=kv_dtype,
                            q_dtype=q_dtype, seed=40 + D + Hq)
     check_close(got, ref, **tol_for(kv_dtype), what=f"keys split over waves kv={kv_dtype} D={D} G={Hq // Hkv}")
@@ -286,6 +304,8 @@ def test_prefill_keys_split_over_waves(stream, kv_dtype, q_dtype, Hq, Hkv, D, pr
     (0, 16, 16, 32, [0, 20, 300, 7, 0], [150, 260, 16, 1, 250]),  # four
     (1, 8, 8, 32, [5] * 15 + [200], [400] * 15 + [391]),       # two
     (0, 9, 3, 32, [0] * 40, [481] + [353] * 39),               # one
+    (0, 4, 4, 64, [5, 300, 77], [33, 20, 3]),                  # 12 (sequence, KV head) groups: 8 and a remainder
+    (1, 3, 1, 128, [0, 20, 7, 64, 3, 40, 1, 90, 15, 16, 200], [17] * 11),      # 11
     (0, 4, 2, 256, [70, 0, 300], [33, 16, 120]),
 ])
 def test_prefill_fp32_waves_per_unit(stream, q_dtype, Hq, Hkv, D, prefix, chunk):
