@@ -11,12 +11,11 @@
 //
 // Work decomposition: a unit is one 16-query tile of one query head. A wave computes NU = 2 units of
 // one (sequence, KV head) on the same K/V operands, one from either end of the tile order, so that
-// under the causal mask every pair has about the same work; or one unit (head_dim 256, and calls
-// of at most one unit per CU). KS waves share their keys: wave i of them takes blocks i, i + KS, ..,
-// and at the end the waves leave their (max, sum, O) in LDS and add them up, each a part of the
-// output dims. KS is the smallest of 1, 2, 4, 8 that gives every SIMD of the chip two waves (one for
-// head_dim 256): a wave is one serial chain over its blocks (products, softmax, products) and a
-// second one fills its gaps.
+// under the causal mask every pair has about the same work; or one unit (head_dim 256, calls of at most
+// one unit per CU, and chunks of few tiles). KS waves share their keys: wave i of them takes blocks i, i + KS,
+// .., and at the end the waves leave their (max, sum, O) in LDS and add them up, each a part of the
+// output dims. A workgroup has 4 waves, and two of them fit a CU (one for head_dim 256), or the 8 of KS = 8.
+// KS is the number for which generations of workgroups times a wave's blocks are least.
 //
 // A wave's blocks come one at a time into an LDS slot of its own (LDS-direct loads of whole lines;
 // operands loaded straight into registers held the kernel at 42 us where this one takes 31): the
@@ -114,14 +113,15 @@ __device__ __forceinline__ void lds_load_segments(u32x4_t r, const uint32_t* off
     }
 }
 
-// Waves of a workgroup: 8, or the 4 whose slots of head_dim 256 fit the LDS.
-__host__ __device__ constexpr int f32_waves(int d) { return d > 128 ? 4 : 8; }
+// Waves of a workgroup: 4, or the 8 that share a unit's keys; and workgroups a CU's LDS holds (head_dim 256: one).
+__host__ __device__ constexpr int f32_waves(int ks) { return ks > 4 ? 8 : 4; }
+__host__ __device__ constexpr int f32_per_cu(int d, int ks) { return d > 128 || ks > 4 ? 1 : 2; }
 
 template <int D, int KS, int NU>
-__global__ __launch_bounds__((64 * f32_waves(D)), (f32_waves(D) / 4)) void chunked_prefill_fp32_kernel(const PrefillF32Args a) {
+__global__ __launch_bounds__((64 * f32_waves(KS)), (f32_waves(KS) / 4 * f32_per_cu(D, KS))) void chunked_prefill_fp32_kernel(const PrefillF32Args a) {
     using TL = F32Tile<D>;
     constexpr int NT = D / 16;  // 16-dim slabs of K and output tiles
-    constexpr int WAVES = f32_waves(D);
+    constexpr int WAVES = f32_waves(KS);
     constexpr int SEG = TL::SEG;
     // The waves' slots, reused for their states.
     __shared__ uint4 s_tile[WAVES * 2 * TL::CHUNKS];
@@ -295,58 +295,63 @@ __global__ __launch_bounds__((64 * f32_waves(D)), (f32_waves(D) / 4)) void chunk
     };
     auto stored = [&](int k) { return nblk[k] > 0 && i0[k] + n < Lc; };
     if constexpr (KS > 1) {
-        // Every wave leaves its state in its own slot; piece i (unit i / NT, dims 16 (i % NT) .. + 15) of a
-        // set is added up and stored by wave i % KS of it.
+        // Every wave with keys leaves its state in its own slot; piece i (unit i / NT, dims 16 (i % NT) .. + 15)
+        // of a set is added up and stored by wave i % KS of it.
+        const int busy = min(KS, nkb);
 #pragma unroll
         for (int k = 0; k < NU; k++) {
+            if (ks >= busy || busy == 1) break;
             s_ml[(wave * NU + k) * 64 + lane] = make_float2(m_run[k], l_run[k]);
 #pragma unroll
             for (int t = 0; t < NT; t++)
                 s_tile[wave * 2 * TL::CHUNKS + (k * NT + t) * 64 + lane] = __builtin_bit_cast(uint4, acc[k][t]);
         }
         __syncthreads();
-        const int w0 = uw * KS;
+        if (busy != 1) {
+            const int w0 = uw * KS;
 #pragma unroll
-        for (int k = 0; k < NU; k++) {
-            if (nblk[k] == 0) continue;
-            float2 ml[KS];
-            float mt = -__FLT_MAX__;
+            for (int k = 0; k < NU; k++) {
+                if (nblk[k] == 0) continue;
+                float2 ml[KS];
+                float mt = -__FLT_MAX__;
 #pragma unroll
-            for (int i = 0; i < KS; i++) {
-                ml[i] = s_ml[((w0 + i) * NU + k) * 64 + lane];
-                mt = fmaxf(mt, ml[i].x);
+                for (int i = 0; i < KS; i++) {
+                    ml[i] = i < busy ? s_ml[((w0 + i) * NU + k) * 64 + lane] : make_float2(-__FLT_MAX__, 0.0f);
+                    mt = fmaxf(mt, ml[i].x);
+                }
+                float l = 0.0f, f[KS];
+#pragma unroll
+                for (int i = 0; i < KS; i++) {
+                    f[i] = __builtin_amdgcn_exp2f(ml[i].x - mt);
+                    l += ml[i].y * f[i];
+                }
+                const float inv = 1.0f / rows_sum(l);  // lanes n, n + 16, .. held partial sums of query n
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    if ((k * NT + t) % KS != ks) continue;
+                    f32x4_t o = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int i = 0; i < KS; i++)
+                        if (i < busy) o += __builtin_bit_cast(f32x4_t, s_tile[(w0 + i) * 2 * TL::CHUNKS + (k * NT + t) * 64 + lane]) * f[i];
+                    if (stored(k)) *reinterpret_cast<f32x4_t*>(out_row(k) + 16 * t) = o * inv;
+                }
             }
-            float l = 0.0f, f[KS];
-#pragma unroll
-            for (int i = 0; i < KS; i++) {
-                f[i] = __builtin_amdgcn_exp2f(ml[i].x - mt);
-                l += ml[i].y * f[i];
-            }
-            const float inv = 1.0f / rows_sum(l);  // lanes n, n + 16, .. held partial sums of query n
-#pragma unroll
-            for (int t = 0; t < NT; t++) {
-                if ((k * NT + t) % KS != ks) continue;
-                f32x4_t o = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int i = 0; i < KS; i++)
-                    o += __builtin_bit_cast(f32x4_t, s_tile[(w0 + i) * 2 * TL::CHUNKS + (k * NT + t) * 64 + lane]) * f[i];
-                if (stored(k)) *reinterpret_cast<f32x4_t*>(out_row(k) + 16 * t) = o * inv;
-            }
+            return;
         }
-    } else {
+        if (ks > 0) return;  // one block of keys: wave 0 of the set has it all
+    }
 #pragma unroll
-        for (int k = 0; k < NU; k++) {
-            const float inv = 1.0f / rows_sum(l_run[k]);
-            if (!stored(k)) continue;
+    for (int k = 0; k < NU; k++) {
+        const float inv = 1.0f / rows_sum(l_run[k]);
+        if (!stored(k)) continue;
 #pragma unroll
-            for (int t = 0; t < NT; t++) *reinterpret_cast<f32x4_t*>(out_row(k) + 16 * t) = acc[k][t] * inv;
-        }
+        for (int t = 0; t < NT; t++) *reinterpret_cast<f32x4_t*>(out_row(k) + 16 * t) = acc[k][t] * inv;
     }
 }
 
 template <int D>
 void launch_ks(const PrefillF32Args& a, int nu, int ks, dim3 grid, hipStream_t s) {
-    constexpr int threads = 64 * f32_waves(D);
+    const int threads = 64 * f32_waves(ks);
     if constexpr (D > 128) {
         switch (ks) {
             case 1: chunked_prefill_fp32_kernel<D, 1, 1><<<grid, threads, 0, s>>>(a); break;
@@ -354,7 +359,12 @@ void launch_ks(const PrefillF32Args& a, int nu, int ks, dim3 grid, hipStream_t s
             default: chunked_prefill_fp32_kernel<D, 4, 1><<<grid, threads, 0, s>>>(a); break;
         }
     } else if (nu == 1) {
-        chunked_prefill_fp32_kernel<D, 8, 1><<<grid, threads, 0, s>>>(a);
+        switch (ks) {
+            case 1: chunked_prefill_fp32_kernel<D, 1, 1><<<grid, threads, 0, s>>>(a); break;
+            case 2: chunked_prefill_fp32_kernel<D, 2, 1><<<grid, threads, 0, s>>>(a); break;
+            case 4: chunked_prefill_fp32_kernel<D, 4, 1><<<grid, threads, 0, s>>>(a); break;
+            default: chunked_prefill_fp32_kernel<D, 8, 1><<<grid, threads, 0, s>>>(a); break;
+        }
     } else {
         switch (ks) {
             case 1: chunked_prefill_fp32_kernel<D, 1, 2><<<grid, threads, 0, s>>>(a); break;
@@ -388,14 +398,26 @@ pa_status launch_chunked_prefill_fp32(hipStream_t s, const pa_config* cfg, float
     a.q_bf16 = cfg->q_dtype == PA_DTYPE_BF16;
     const int64_t ng = static_cast<int64_t>(num_seqs) * cfg->num_kv_heads;
     const int64_t units = static_cast<int64_t>(a.group) * ((static_cast<int64_t>(max_chunk_len) + 15) / 16);
-    const int waves = f32_waves(cfg->head_dim);
-    // One unit a wave while every unit can have a CU (100 queries, 8 heads of 128: 7.8 us against 11.8),
-    // two beyond (8 x 512 on 350 tokens: 92 against 124 us).
-    const int nu = cfg->head_dim > 128 || ng * units <= device_cus() ? 1 : 2;
-    int ks = 1;
-    while (ks < waves && ng * ((units + nu - 1) / nu) * ks < waves * device_cus()) ks *= 2;
+    // One unit a wave while every unit can have a CU, and for chunks of few tiles (40 x 33 tokens, 16 / 4 heads of 128:
+    // 13.5 us against 17.2; 16 x 100: 20.4 against 22.3); two beyond (16 x 128: 23.7 against 26.0; 8 x 512: 88 against
+    // 102; 2 x 512 on 350: 52.6 against 54.7).
+    const int64_t tiles = units / a.group;
+    const int nu = cfg->head_dim > 128 || ng * units <= device_cus() || tiles < 8 ? 1 : 2;
     const int64_t sets = (units + nu - 1) / nu;  // per (sequence, KV head)
-    const int64_t wpg = (sets + waves / ks - 1) / (waves / ks);
+    // Waves on a set's keys: the number with the least generations of workgroups times (a constant part, the
+    // launch, first loads and the exchange, about two and a half blocks, and a wave's blocks; the table's width bounds them).
+    auto groups = [&](int n) { return (sets + f32_waves(n) / n - 1) / (f32_waves(n) / n); };
+    int ks = 1;
+    int64_t least = 0;
+    for (int n = 1; n <= (cfg->head_dim > 128 ? 4 : 8); n *= 2) {
+        const int64_t hold = static_cast<int64_t>(f32_per_cu(cfg->head_dim, n)) * device_cus();
+        const int64_t cost = (ng * groups(n) + hold - 1) / hold * (5 + 2 * ((max_blocks_per_seq + n - 1) / n));
+        if (n == 1 || cost <= least) {
+            ks = n;
+            least = cost;
+        }
+    }
+    const int64_t wpg = groups(ks);
     const int64_t nwg = placed_grid(ng, wpg);
     if (nwg > 0x7fffffff) return set_error(PA_ERROR_UNSUPPORTED, "pa_chunked_prefill: grid too large");
     a.wg_per_group = static_cast<int32_t>(wpg);

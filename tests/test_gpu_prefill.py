@@ -301,8 +301,15 @@ def test_prefill_keys_split_over_waves(stream, kv_dtype, q_dtype, Hq, Hkv, D, pr
     (0, 6, 2, 64, [333, 0], [17, 1]),                          # an odd number of units; one unit a wave
     (1, 1, 1, 128, [16 * 64 * 8 - 3, 0], [3, 16]),             # more than 64 blocks a wave
     (0, 8, 8, 64, [100, 0, 31], [130, 305, 16]),               # two units a wave, eight waves on their keys
-    (0, 16, 16, 32, [0, 20, 300, 7, 0], [150, 260, 16, 1, 250]),  # four
-    (1, 8, 8, 32, [5] * 15 + [200], [400] * 15 + [391]),       # two
+    (0, 16, 16, 32, [0, 20, 300, 7, 0], [150, 260, 16, 1, 250]),  # two
+    (0, 16, 16, 64, [0, 3, 16, 0, 40], [150, 16, 17, 1, 100]),  # four
+    (1, 8, 8, 32, [5] * 15 + [200], [400] * 15 + [391]),       # one
+    (1, 8, 8, 128, [5, 0, 200, 3, 0, 7, 16, 1], [400, 16, 33, 250, 1, 90, 17, 399]),  # two
+    # one unit a wave: one, two, four waves on its keys
+    (0, 16, 8, 128, [0, 3, 20] * 8, [60, 16, 33] * 8),
+    (1, 8, 8, 32, [3, 0, 30, 1] * 16, [20, 1, 16, 17] * 16),
+    (0, 16, 16, 64, [60, 0, 3, 16] * 2, [33, 16, 1, 40] * 2),
+    (0, 4, 4, 256, [40, 0] * 20, [33, 16] * 20),
     (0, 9, 3, 32, [0] * 40, [481] + [353] * 39),               # one
     (0, 4, 4, 64, [5, 300, 77], [33, 20, 3]),                  # 12 (sequence, KV head) groups: 8 and a remainder
     (1, 3, 1, 128, [0, 20, 7, 64, 3, 40, 1, 90, 15, 16, 200], [17] * 11),      # 11
