@@ -578,12 +578,18 @@ LONG_LENS = [5000, 1, 4100, 3000, 17, 6000, 40000, 1025, 2049]
     (2, 1, 8, 2, 256, 512, APPEND_LENS), (0, 0, 8, 8, 64, 256, APPEND_LENS), (0, 1, 16, 4, 128, 512, APPEND_LENS),
     (1, 1, 16, 4, 128, 256, APPEND_LENS), (1, 1, 8, 2, 128, 4096, LONG_LENS), (2, 1, 8, 2, 128, 0, LONG_LENS),
     (1, 1, 32, 8, 128, 0, TAIL_LENS), (2, 0, 32, 8, 128, 0, TAIL_LENS),
-    # one range, no merge launch: the owning wave writes the token (V tile patched in LDS)
-    (1, 1, 32, 8, 128, 0, [40]), (1, 0, 8, 2, 64, -1, [1000]), (1, 1, 8, 2, 128, -1, [33]), (1, 1, 16, 4, 256, 0, [64]),
+    # ranges and a merge launch at every position
+    (1, 1, 32, 8, 128, 64, TAIL_LENS), (1, 0, 16, 4, 64, -2, TAIL_LENS), (1, 0, 8, 8, 32, 64, TAIL_LENS),
+    (1, 1, 16, 2, 256, 0, TAIL_LENS), (2, 0, 32, 8, 128, 64, TAIL_LENS),
+    # one sequence, one range, no merge launch: the owning wave writes the token (V tile patched in LDS)
+    (1, 1, 32, 8, 128, 64, [40]), (1, 0, 8, 2, 64, -1, [1000]), (1, 1, 8, 2, 128, -1, [33]), (1, 1, 16, 4, 256, 0, [64]),
+    # one sequence of a workgroup per row, which writes it itself
+    (1, 1, 32, 8, 128, 0, [40]), (1, 0, 8, 2, 64, 0, [1]), (1, 1, 4, 2, 32, 0, [17]),
     (1, 1, 8, 2, 64, 0, MANY_LENS), (2, 0, 8, 2, 64, 0, MANY_LENS),
 ], ids=["bf16-split16", "int8-split5", "bf16-auto", "bf16-d64", "int8-auto", "int8-d256", "fp32-d64", "fp32-d128", "bf16-256", "bf16-long",
-        "int8-long", "bf16-tails", "int8-tails", "bf16-one-range", "bf16-one-split", "bf16-one-split-new-block",
-        "bf16-one-range-d256", "bf16-many-seqs", "int8-many-seqs"])
+        "int8-long", "bf16-tails", "int8-tails", "bf16-tails-ranges", "bf16-tails-splits", "bf16-tails-ranges-d32",
+        "bf16-tails-d256", "int8-tails-ranges", "bf16-one-range", "bf16-one-split", "bf16-one-split-new-block",
+        "bf16-one-range-d256", "bf16-one-row", "bf16-one-row-first-token", "bf16-one-row-d32", "bf16-many-seqs", "int8-many-seqs"])
 def test_decode_append_matches_append_then_decode(stream, kv_dtype, q_dtype, Hq, Hkv, D, part, lens):
     w = wl.make_small(70 + D + kv_dtype, num_seqs=len(lens), lens=lens, Hq=Hq, Hkv=Hkv, D=D,
                       kv_dtype=kv_dtype, q_dtype=q_dtype)
@@ -673,6 +679,78 @@ def test_decode_short_rows(stream, kv_dtype, q_dtype, Hq, Hkv, D, lens):
     check_close(got, ref, **tol_for(kv_dtype), what=f"short rows kv={kv_dtype} D={D} G={Hq // Hkv}")
     assert np.all(got[-1] == 0.0)
     test_decode_append_matches_append_then_decode(stream, kv_dtype, q_dtype, Hq, Hkv, D, 0, lens)
+
+
+@pytest.mark.parametrize("part", [0, 64])
+@pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D", [(1, 1, 32, 8, 128), (1, 0, 4, 2, 32), (2, 0, 16, 4, 64), (2, 1, 8, 8, 128)])
+def test_decode_short_rows_invalid_block_ids(stream, kv_dtype, q_dtype, Hq, Hkv, D, part):
+    """Block ids below 0 and past the pool, in blocks that are read (zeros) and in the one a token is appended to
+    (not stored; the token is attended to): plain and fused, a workgroup per row and (part) ranges with a
+    merge. Everything else in the cache stays as it is."""
+    lens = [1, 1, 16, 17, 40, 100, 300, 300, 500, 33]
+    w = wl.make_small(960 + D, num_seqs=len(lens), lens=lens, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=kv_dtype, q_dtype=q_dtype)
+    bad = w.num_blocks + 3
+    w.block_tables[0, 0] = -1   # the only token's block
+    w.block_tables[3, 1] = bad  # a block of the new token alone
+    w.block_tables[4, 0] = -5
+    w.block_tables[5, 6] = -1   # the last block, streamed in part
+    w.block_tables[6, 18] = bad
+    w.block_tables[7, 3], w.block_tables[7, 11] = -1, bad
+    w.block_tables[9, :] = -1   # none of its blocks
+    got, ref = run_decode(w, 82, stream, partition_size=part)
+    check_close(got, ref, **tol_for(kv_dtype), what=f"invalid ids kv={kv_dtype} D={D} part={part}")
+    inp = wl.numpy_inputs(w, 83)
+    cfg = config_for(w, partition_size=part)
+    S = w.num_seqs
+    rng = np.random.default_rng(84)
+    k_new, v_new = (rng.standard_normal((S, Hkv, D), dtype=np.float32) for _ in "kv")
+    if q_dtype == 1:
+        k_new, v_new = orc.bf16_from_f32(k_new), orc.bf16_from_f32(v_new)
+    pos = w.context_lens.astype(np.int64) - 1
+    blk = w.block_tables[np.arange(S), pos // 16].astype(np.int64)
+    slots = np.where((blk >= 0) & (blk < w.num_blocks), blk * 16 + pos % 16, -1)
+    stats = [None] * 4
+    if kv_dtype == 2:
+        host, g = build_int8_caches(w, inp, stream)
+        kc, vc = g["kc"], g["vc"]
+        stats = [g["ks"], g["vs"], g["ka"], g["va"]]
+        hk, hv = host["k_cache"].copy(), host["v_cache"].copy()
+        hstats = [to_np(t).copy() for t in stats]
+        orc.kv_append(cfg, k_new, v_new, slots, hk, hv, *hstats)
+    else:
+        kc, vc = to_gpu(inp["k_cache"]), to_gpu(inp["v_cache"])
+        hk, hv = inp["k_cache"].copy(), inp["v_cache"].copy()
+        hstats = [None] * 4
+        orc.kv_append(cfg, k_new, v_new, slots, hk, hv)
+    out = empty_gpu((S, Hq, D), np.float32)
+    out.fill_(float("nan"))
+    wsb = pa.decode_workspace_size(cfg, S, w.max_context_len)
+    ws = empty_gpu((max(wsb, 1),), np.uint8)
+    pa.paged_decode_append(stream, cfg, out, to_gpu(inp["q"]), to_gpu(k_new), to_gpu(v_new), kc, vc, *stats,
+                           to_gpu(w.block_tables), to_gpu(w.context_lens), S, w.max_blocks, w.max_context_len, ws, wsb)
+    _sync()
+    cdt = {1: np.uint16, 2: np.int8}[kv_dtype]
+    np.testing.assert_array_equal(to_np(kc, cdt), hk)
+    np.testing.assert_array_equal(to_np(vc, cdt), hv)
+    for t, want in zip(stats, hstats):
+        if t is not None:
+            np.testing.assert_array_equal(to_np(t), want)
+    ref = orc.paged_decode(cfg, inp["q"], hk, hv, hstats[0], hstats[1], w.block_tables, w.context_lens, n_threads=NTHREADS)
+    stored = slots >= 0
+    check_close(to_np(out)[stored], ref[stored], **tol_for(kv_dtype), what="fused, invalid ids")
+    if kv_dtype == 1:  # the new token joins from k_new / v_new, whether its block can hold it or not
+        full = w.block_tables.copy()
+        unused = np.setdiff1d(np.arange(w.num_blocks), w.block_tables)
+        full[~stored, pos[~stored] // 16] = unused[:(~stored).sum()]
+        k1, v1 = inp["k_cache"].copy(), inp["v_cache"].copy()
+        for s in np.nonzero(~stored)[0]:
+            b = full[s, pos[s] // 16]
+            k1.reshape(w.num_blocks, Hkv, 16, D)[b] = 0
+            v1.reshape(w.num_blocks, Hkv, D, 16)[b] = 0
+        orc.kv_append(cfg, k_new, v_new, np.where(stored, -1, full[np.arange(S), pos // 16].astype(np.int64) * 16 + pos % 16),
+                      k1, v1)
+        ref = orc.paged_decode(cfg, inp["q"], k1, v1, None, None, full, w.context_lens, n_threads=NTHREADS)
+        check_close(to_np(out)[~stored], ref[~stored], **tol_for(1), what="fused, the new token's block invalid")
 
 
 @pytest.mark.parametrize("D,base,S,part", [

@@ -71,13 +71,15 @@ PREFIX = [0, 1, 15, 16, 17, 37, 300, 1000]
 CHUNK = [33, 1, 16, 17, 100, 64, 5, 130]
 
 
+# Three of each make more workgroups than the key-split kernel takes: the waves share one stream of keys.
+@pytest.mark.parametrize("copies", [1, 3])
 @pytest.mark.parametrize("flags", [0, pa.PA_FLAG_REFERENCE_LITERAL_MASK, pa.PA_FLAG_NO_MASK])
 @pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D", [
     (1, 1, 32, 8, 128), (1, 0, 8, 8, 64), (2, 1, 16, 2, 128), (2, 0, 8, 1, 64), (1, 1, 8, 4, 256),
     (2, 1, 8, 2, 256),
 ])
-def test_prefill_ragged(stream, flags, kv_dtype, q_dtype, Hq, Hkv, D):
-    got, ref = run_prefill(stream, prefix=PREFIX, chunk=CHUNK, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=kv_dtype,
+def test_prefill_ragged(stream, flags, kv_dtype, q_dtype, Hq, Hkv, D, copies):
+    got, ref = run_prefill(stream, prefix=PREFIX * copies, chunk=CHUNK * copies, Hq=Hq, Hkv=Hkv, D=D, kv_dtype=kv_dtype,
                            q_dtype=q_dtype, flags=flags, seed=D + kv_dtype)
     check_close(got, ref, **tol_for(kv_dtype), what=f"prefill flags={flags} kv={kv_dtype} D={D} G={Hq // Hkv}")
 
@@ -115,14 +117,20 @@ def test_prefill_empty_chunks_and_single_query(stream):
     check_close(got, ref, **tol_for(1), what="empty chunks")
 
 
-def test_prefill_invalid_block_ids_read_as_zero(stream):
+@pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D,copies", [
+    (1, 0, 8, 2, 64, 1), (2, 1, 16, 4, 128, 1),     # one and two units a workgroup of the key-split kernel
+    (1, 1, 32, 8, 128, 3), (2, 0, 32, 8, 64, 3),    # four
+    (1, 1, 32, 8, 128, 8), (2, 1, 32, 8, 64, 8),    # the waves share one stream of keys
+])
+def test_prefill_invalid_block_ids_read_as_zero(stream, kv_dtype, q_dtype, Hq, Hkv, D, copies):
     def edit(w):
         w.block_tables[0, 2] = -1
         w.block_tables[1, 1] = w.num_blocks + 3
+        w.block_tables[1, 20] = -7
 
-    got, ref = run_prefill(stream, prefix=[40, 20], chunk=[30, 50], Hq=8, Hkv=2, D=64, kv_dtype=1, q_dtype=0,
-                           seed=4, table_edit=edit)
-    check_close(got, ref, **tol_for(1), what="invalid ids")
+    got, ref = run_prefill(stream, prefix=[40, 320] * copies, chunk=[30, 50] * copies, Hq=Hq, Hkv=Hkv, D=D,
+                           kv_dtype=kv_dtype, q_dtype=q_dtype, seed=4, table_edit=edit)
+    check_close(got, ref, **tol_for(kv_dtype), what="invalid ids")
 
 
 def test_prefill_c3_shape(stream):
@@ -181,11 +189,22 @@ def _scale_v(factor):
 
 
 @pytest.mark.parametrize("flags", [0, pa.PA_FLAG_REFERENCE_LITERAL_MASK, pa.PA_FLAG_NO_MASK])
-@pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D,edit", [
-    (1, 1, 32, 8, 128, _bf16_outliers), (1, 0, 8, 2, 64, _bf16_outliers),
-    (1, 1, 32, 8, 128, _scale_v(2.0 ** 16)), (2, 1, 16, 4, 128, _scale_v(4096.0)), (2, 0, 8, 8, 64, _scale_v(4096.0)),
-], ids=["bf16-outliers", "bf16-outliers-d64", "bf16-x65536", "int8-x4096", "int8-x4096-d64"])
-def test_prefill_values_beyond_fp16_range(stream, flags, kv_dtype, q_dtype, Hq, Hkv, D, edit):
+@pytest.mark.parametrize("kv_dtype,q_dtype,Hq,Hkv,D,edit,copies", [
+    (1, 1, 32, 8, 128, _bf16_outliers, 1), (1, 0, 8, 2, 64, _bf16_outliers, 1),
+    (1, 1, 32, 8, 128, _scale_v(2.0 ** 16), 1), (2, 1, 16, 4, 128, _scale_v(4096.0), 1),
+    (2, 0, 8, 8, 64, _scale_v(4096.0), 1),
+    # the most units a workgroup of the key-split kernel takes
+    (1, 1, 32, 8, 128, _bf16_outliers, 2), (1, 0, 8, 2, 64, _bf16_outliers, 6), (1, 1, 8, 2, 256, _bf16_outliers, 3),
+    (2, 1, 16, 4, 128, _scale_v(4096.0), 3),
+    # more workgroups than it takes: the waves share one stream of keys; 16 heads a group are two rounds of units
+    (1, 1, 32, 8, 128, _bf16_outliers, 5), (1, 0, 8, 2, 64, _bf16_outliers, 18), (1, 0, 16, 1, 128, _bf16_outliers, 10),
+    (1, 1, 32, 8, 128, _scale_v(2.0 ** 16), 5), (2, 1, 16, 4, 128, _scale_v(4096.0), 10),
+    (2, 0, 8, 8, 64, _scale_v(4096.0), 20),
+], ids=["bf16-outliers", "bf16-outliers-d64", "bf16-x65536", "int8-x4096", "int8-x4096-d64", "bf16-outliers-most",
+        "bf16-outliers-d64-most", "bf16-outliers-d256-most", "int8-x4096-most", "bf16-outliers-stream",
+        "bf16-outliers-d64-stream", "bf16-outliers-g16-stream", "bf16-x65536-stream", "int8-x4096-stream",
+        "int8-x4096-d64-stream"])
+def test_prefill_values_beyond_fp16_range(stream, flags, kv_dtype, q_dtype, Hq, Hkv, D, edit, copies):
     """V magnitudes past fp16's 65504.
     bf16 outliers: 0.3 % of V entries at +-[65536, 1e5) among N(0,1) values, at the unchanged bar
     (an output dim mixes only that dim's V values, so the outliers' dims are held to 1e-2 of their
@@ -193,8 +212,8 @@ def test_prefill_values_beyond_fp16_range(stream, flags, kv_dtype, q_dtype, Hq, 
     far past fp16): attention is linear in V and the factor is exact, so outputs divided by the
     factor are held to the unit-scale bar -- the bar the errors of fp16 / bf16 probabilities scale
     with."""
-    got, ref = run_prefill(stream, prefix=[0, 17, 300, 40], chunk=[40, 33, 64, 1], Hq=Hq, Hkv=Hkv, D=D,
-                           kv_dtype=kv_dtype, q_dtype=q_dtype, flags=flags, seed=11 + D + kv_dtype,
+    got, ref = run_prefill(stream, prefix=[0, 17, 300, 40] * copies, chunk=[40, 33, 64, 1] * copies, Hq=Hq, Hkv=Hkv,
+                           D=D, kv_dtype=kv_dtype, q_dtype=q_dtype, flags=flags, seed=11 + D + kv_dtype,
                            input_edit=edit)
     f = getattr(edit, "factor", 1.0)
     assert np.abs(ref).max() > 1000.0, "the case must reach large outputs"
