@@ -785,7 +785,7 @@ __global__ __launch_bounds__(kPrefillThreads, D > 128 ? 1 : (D > 64 && QF32 ? 2 
 // What bounds it: with NU = 4, VALU issue (softmax, V conversion) and MFMA, which two waves a SIMD
 // overlap only in part: about 2300 clocks per pair and wave against 1400 of VALU and 1020 of MFMA. A
 // 512-token chunk on 3333 tokens, Llama shape (32 / 8 heads of 128, bf16): 109.5 -> 46 us (660
-// TFLOP/s); int8 cache, 512 on 2000: 109 -> 43. (The instances of head_dim 128 and bf16 queries spill 13
+// TFLOP/s); int8 cache, 512 on 2000: 109 -> 43. (The instances of head_dim 128 and bf16 queries spill 14
 // registers, 41 over int8 caches, whose reloads the compiler waits for in the counter that the loop's own
 // loads share: in part they undo the prefetch.) With few units, the loads through LDS, and for short
 // contexts the launch and its round trips: 20 tokens on 8000 217 -> 39 us (71 with NU = 4), 203 tokens
@@ -1297,14 +1297,14 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32, NU>()), (wave_waves<D, QF
             if (qi < nq[k]) {
                 const float l = __shfl(l_tot, qi, 64);
                 const float inv = 1.0f / l;
-                const bool sum_ok = (__float_as_uint(l) & 0x7f800000u) != 0x7f800000u;
+                uint32_t top = 0;  // of the row's magnitudes, as bits: one test a row (one a value cost the kernel 2%)
                 float* op = a.out + (static_cast<int64_t>(q0 + i0[k] + qi) * Hq + head[k]) * D;
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
-                    if constexpr (ELT == 2)
-                        bad = bad || (sum_ok && (__float_as_uint(acc[k][t][i]) & 0x7f800000u) == 0x7f800000u);
+                    if constexpr (ELT == 2) top = max(top, __float_as_uint(acc[k][t][i]) & 0x7fffffffu);
                     op[16 * t + n] = acc[k][t][i] * inv;
                 }
+                if constexpr (ELT == 2) bad = bad || (top >= 0x7f800000u && (__float_as_uint(l) & 0x7f800000u) != 0x7f800000u);
             }
         }
         if constexpr (ELT == 2) {
