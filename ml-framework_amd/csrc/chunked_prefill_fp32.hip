@@ -295,19 +295,18 @@ __global__ __launch_bounds__((64 * f32_waves(KS)), (f32_waves(KS) / 4 * f32_per_
     };
     auto stored = [&](int k) { return nblk[k] > 0 && i0[k] + n < Lc; };
     if constexpr (KS > 1) {
-        // Every wave with keys leaves its state in its own slot; piece i (unit i / NT, dims 16 (i % NT) .. + 15)
-        // of a set is added up and stored by wave i % KS of it.
-        const int busy = min(KS, nkb);
+        // Every wave leaves its state in its own slot; piece i (unit i / NT, dims 16 (i % NT) .. + 15) of a set is
+        // added up and stored by wave i % KS of it.
 #pragma unroll
         for (int k = 0; k < NU; k++) {
-            if (ks >= busy || busy == 1) break;
+            if (nkb == 1) break;
             s_ml[(wave * NU + k) * 64 + lane] = make_float2(m_run[k], l_run[k]);
 #pragma unroll
             for (int t = 0; t < NT; t++)
                 s_tile[wave * 2 * TL::CHUNKS + (k * NT + t) * 64 + lane] = __builtin_bit_cast(uint4, acc[k][t]);
         }
         __syncthreads();
-        if (busy != 1) {
+        if (nkb != 1) {
             const int w0 = uw * KS;
 #pragma unroll
             for (int k = 0; k < NU; k++) {
@@ -316,7 +315,7 @@ __global__ __launch_bounds__((64 * f32_waves(KS)), (f32_waves(KS) / 4 * f32_per_
                 float mt = -__FLT_MAX__;
 #pragma unroll
                 for (int i = 0; i < KS; i++) {
-                    ml[i] = i < busy ? s_ml[((w0 + i) * NU + k) * 64 + lane] : make_float2(-__FLT_MAX__, 0.0f);
+                    ml[i] = s_ml[((w0 + i) * NU + k) * 64 + lane];
                     mt = fmaxf(mt, ml[i].x);
                 }
                 float l = 0.0f, f[KS];
@@ -332,7 +331,7 @@ __global__ __launch_bounds__((64 * f32_waves(KS)), (f32_waves(KS) / 4 * f32_per_
                     f32x4_t o = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                     for (int i = 0; i < KS; i++)
-                        if (i < busy) o += __builtin_bit_cast(f32x4_t, s_tile[(w0 + i) * 2 * TL::CHUNKS + (k * NT + t) * 64 + lane]) * f[i];
+                        o += __builtin_bit_cast(f32x4_t, s_tile[(w0 + i) * 2 * TL::CHUNKS + (k * NT + t) * 64 + lane]) * f[i];
                     if (stored(k)) *reinterpret_cast<f32x4_t*>(out_row(k) + 16 * t) = o * inv;
                 }
             }
