@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Paged-attention benchmark on one MI355X (the BASELINE.json metric, plus the other configurations).
+"""Paged-attention benchmark on one MI355X (the headline metric, plus the other configurations).
 
 Headline step = one decode layer-step of the C2 configuration (Llama-3-8B layer shape: Hq=32,
 Hkv=8, D=128, bf16 KV, block 16, batch 64, contexts log-uniform in [128, 4096], shuffled physical

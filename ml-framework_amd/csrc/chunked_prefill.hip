@@ -1297,7 +1297,7 @@ __global__ __launch_bounds__((64 * wave_waves<D, QF32, NU>()), (wave_waves<D, QF
             if (qi < nq[k]) {
                 const float l = __shfl(l_tot, qi, 64);
                 const float inv = 1.0f / l;
-                uint32_t top = 0;  // of the row's magnitudes, as bits: one test a row (one a value cost the kernel 2%)
+                uint32_t top = 0;  // the row's largest magnitude, as bits: one test a row (one a value cost the kernel 2%)
                 float* op = a.out + (static_cast<int64_t>(q0 + i0[k] + qi) * Hq + head[k]) * D;
 #pragma unroll
                 for (int t = 0; t < NT; t++) {

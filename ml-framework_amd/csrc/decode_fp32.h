@@ -1,4 +1,4 @@
-// decode_fp32.h -- the fp32-cache paged-decode kernel (VALU).
+// decode_fp32.h -- the fp32-cache paged-decode kernels: VALU for groups of 1 and 2 query heads, matrix for 4 and 8.
 #pragma once
 
 #include "decode_common.h"

@@ -10,10 +10,15 @@
 // streams the same bytes whatever the mix of context lengths; rows (sequence, KV head) split
 // between ranges leave (max, sum, unnormalised O) partials that paged_decode_merge_split_kernel
 // combines with a log-sum-exp reduction. The G = Hq / Hkv query heads of a KV head share every
-// K/V byte loaded (GQA): QK and PV run on MFMA with the heads as the 16 MFMA rows.
-// fp32 caches (decode_fp32.h): one workgroup per (partition, KV head, sequence), VALU dot products
-// reduced across lanes with DPP, a partition-wide softmax in LDS, VALU P.V, and the same kind of
-// merge over fixed 256/512-token partitions (paged_decode_merge_kernel).
+// K/V byte loaded (GQA): QK and PV run on MFMA with the heads as the 16 MFMA rows. Calls of few rows
+// of at most 1024 tokens take paged_decode_mfma_row_kernel instead: a workgroup per (sequence, KV head),
+// no partials and no merge. A fused bf16 append's tokens are written by the merge where one runs, by
+// append_token_bf16_kernel behind the decode where not, or by the decode itself for a single sequence; int8
+// tokens are appended ahead of the decode (append_last_token_int8_kernel).
+// fp32 caches (decode_fp32.h): one workgroup per (partition of 256/512 tokens, KV head, sequence) and the
+// same kind of merge (paged_decode_merge_kernel). Groups of 1 and 2 query heads: VALU dot products
+// reduced across lanes with DPP, a partition-wide softmax in LDS, VALU P.V. Groups of 4 and 8: both
+// products on the 4x4 fp32 MFMA. Tokens are appended ahead of it (append_last_token_fp32_kernel).
 #include <algorithm>
 #include <mutex>
 #include <string>
@@ -48,8 +53,8 @@ constexpr int kMaxNumSplits = 256;
 using pa::clamp_len;
 using pa::act_at;
 
-// Split length for this call. fp32 caches use partitions of 256 or 512 tokens (VALU kernel
-// templates). bf16/int8 caches: 0 lets the kernel cut the batch's blocks into one equal range per
+// Split length for this call. fp32 caches use partitions of 256 or 512 tokens (templates
+// of both kernels). bf16/int8 caches: 0 lets the kernel cut the batch's blocks into one equal range per
 // resident workgroup; otherwise the ranges are `partition_size` tokens (multiple of 64).
 int resolve_part(const pa_config* cfg, std::string* err) {
     const int req = cfg->partition_size;

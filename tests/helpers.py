@@ -10,7 +10,7 @@ import pa_oracle as orc
 BLOCK = 16
 
 # Tolerances of the parity bar: |gpu - oracle| <= atol + rtol * |oracle|, fp32 accumulation.
-# bf16 and int8 caches: the bar north_star states. fp32 caches: the VALU kernel computes in fp32
+# bf16 and int8 caches: the stated parity bar. fp32 caches: the kernels compute in fp32
 # throughout (only the order of the sums and the exp differ from the oracle), so it is held to
 # about 100 fp32 ulps of the outputs' scale.
 TOL_BF16 = dict(atol=2e-3, rtol=1e-2)

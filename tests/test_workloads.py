@@ -1,4 +1,4 @@
-"""Shapes of the seeded benchmark workloads (the five BASELINE.json configurations)."""
+"""Shapes of the seeded benchmark workloads (five configurations)."""
 import numpy as np
 
 import workloads as wl
