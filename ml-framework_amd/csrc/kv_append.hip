@@ -277,14 +277,16 @@ __global__ __launch_bounds__(pa::kAppendMaxThreads) void append_int8_kernel(
 // Latency-bound: the slots, then the run's values and its tile, are two dependent round trips. Against
 // append_int8_block alone, a workgroup a token (whose tokens of a block were applied segment by segment), us
 // of 8 KV heads of 128, bf16: prompt chunks of 4 x 512 210 -> 9.5, of 512 43 -> 7.4, 256 / 1000 decode tokens
-// 9.8 / 31.5 -> 8.9 / 24; 16 prompts of 64 tokens interleaved token by token 64 -> 55; 512 / 1024 tokens in random
-// order 58 / 61 -> 48 / 58 (2048: 64 -> 85, the look over the slots repeated by every workgroup).
+// 9.8 / 31.5 -> 8.9 / 23; 16 prompts of 64 tokens interleaved token by token 64 -> 30; 512 / 1024 tokens in random
+// order 58 / 61 -> 29 / 36 (2048: 64 -> 67, the look over the slots repeated by every workgroup).
 //
-// A window holds one start for a prompt and up to 16 for scattered tokens, which are dealt to gridDim.z
-// workgroups: as many as the chip holds, at least 4 (idle ones cost a prompt little: 4 x 512 tokens 9.5 us with 4
-// or 8, 11 with 16; 256 decode tokens take 12.7 with 4 and 8.9 with 12). With many KV heads a wave takes several pairs:
-// 2048 / n_tok workgroups a window, at least 4 (32 KV heads of 128: 256 decode tokens 15.5 us, with 16 workgroups 24;
-// prompts of 512 14.6 against 10).
+// A window holds one start for a prompt and up to 16 for scattered tokens. Those of them that own their blocks are
+// dealt to gridDim.z workgroups, after the look (dealt before it, two or three blocks of many segments met in
+// one workgroup while others had none: 1024 tokens in random order 58 us against 36): as many as the chip
+// holds, at least 4 (idle ones cost a prompt little: 4 x 512 tokens 9.5 us with 4 or 8, 11 with 16; 256 decode
+// tokens take 12.7 with 4 and 8.9 with 12). With many KV heads a wave takes several pairs: 2048 / n_tok workgroups a
+// window, at least 4 (32 KV heads of 128: 256 decode tokens 15.5 us, with 16 workgroups 24; prompts of 512 14.6
+// against 10).
 constexpr int kRunWaves = 4;
 constexpr int kRunWindow = 16;
 constexpr int kRunPairs = 2048;
@@ -296,6 +298,7 @@ __global__ __launch_bounds__(64 * kRunWaves, D > 128 ? 2 : D > 64 ? 3 : 4) void 
     int64_t capacity, int64_t tok_stride) {
     constexpr int W = kRunWindow;
     __shared__ int s_blk[W], s_len[W], s_other, s_before[W], s_segs[W];
+    __shared__ uint32_t s_map[64];
     __shared__ __align__(16) int8_t s_stage[kRunWaves][pa::kBlockSize * D];
     // A window's workgroups on different XCDs (workgroups are dispatched to the 8 of them in turn).
     const int i0 = static_cast<int>((blockIdx.x + blockIdx.y + gridDim.y * blockIdx.z) % gridDim.x) * W;
@@ -315,61 +318,67 @@ __global__ __launch_bounds__(64 * kRunWaves, D > 128 ? 2 : D > 64 ? 3 : 4) void 
         }
     };
     load_slots(0);
-    const int prev = __shfl_up(blk, 1, 64);
+    const int prev = __shfl_up(blk, 1, 64), prev_row = __shfl_up(row, 1, 64);
     const uint64_t starts = __ballot(lane >= 1 && lane <= W && blk >= 0 && prev != blk);
-    // The starts of a window are dealt to gridDim.z workgroups.
-    uint64_t mine = 0;
-    int rank = 0;
-    for (uint64_t left = starts; left != 0; left &= left - 1, rank++)
-        if (rank % static_cast<int>(gridDim.z) == static_cast<int>(blockIdx.z)) mine |= left & -left;
-    if (mine == 0) return;
-    // Token i0 + w, if it starts a segment: its block and the length of its run of consecutive slots.
-    uint64_t filter = 0;
-    for (uint64_t left = mine; left != 0; left &= left - 1) {
-        const int l = __builtin_ctzll(left);
-        const int b = __builtin_amdgcn_readlane(blk, l), r = __builtin_amdgcn_readlane(row, l);
-        const uint64_t run = __ballot(blk == b && row == r + (lane - l)) >> l;
-        filter |= 1ull << (b & 63);
-        if (tid == 0) {
-            s_blk[l - 1] = b;
-            s_len[l - 1] = __builtin_ctzll(~run);  // at most 16: the run stays in its block
-            s_before[l - 1] = 0;
-            s_segs[l - 1] = 1;
+    // gridDim.z workgroups share a window's blocks; with no more starts than this, none is left for this one.
+    if (__popcll(starts) <= static_cast<int>(blockIdx.z)) return;
+    const uint64_t follows = __ballot(lane >= 1 && blk >= 0 && prev == blk && row == prev_row + 1);
+    // Token i0 + w, if it starts a segment: its block and the length of its run of consecutive slots (at most 16: the
+    // run stays in its block). s_map: by the low six bits of a block, the starts whose block has them.
+    if (wave == 0) {
+        s_map[lane] = 0;
+        __builtin_amdgcn_wave_barrier();
+        if ((starts >> lane) & 1) {
+            const int w = lane - 1;
+            s_blk[w] = blk;
+            s_len[w] = 1 + __builtin_ctzll(~(follows >> (lane + 1)));
+            s_before[w] = 0;
+            s_segs[w] = 1;
+            atomicOr(&s_map[blk & 63], 1u << w);
         }
+        if (lane == 0) s_other = 0;
     }
-    if (tid == 0) s_other = 0;
     __syncthreads();
-    // Bit w of s_other: another token of the call lands in the block that starts at token i0 + w. s_segs[w]: how
-    // many segments of the block the call has; s_before[w]: how many before this one. Slots whose block's low
-    // six bits no such block has are passed over at once.
+    // For w the first start of its block in the window, bit w of s_other: another token of the call lands in the
+    // block. s_segs[w]: how many segments of the block the call has; s_before[w]: how many before this one.
     for (int t0 = 0; t0 < n_tok; t0 += pa::kAppendCoarse * nthreads) {
         if (t0 > 0) load_slots(t0);
 #pragma unroll
         for (int k = 0; k < pa::kAppendCoarse; k++) {
             if (o[k] < 0 || o[k] >= capacity) continue;
             const int b = static_cast<int>(o[k] >> 4), t = t0 + k * nthreads + tid;
-            if (!((filter >> (b & 63)) & 1)) continue;
-            for (uint64_t left = mine; left != 0; left &= left - 1) {
-                const int w = __builtin_ctzll(left) - 1;
-                if (b != s_blk[w] || (t >= i0 + w && t < i0 + w + s_len[w])) continue;
-                atomicOr(&s_other, 1 << w);
-                const int64_t before = t > 0 ? slot_mapping[t - 1] : -1;
-                if (before < 0 || before >= capacity || static_cast<int>(before >> 4) != b) {
-                    atomicAdd(&s_segs[w], 1);
-                    if (t < i0 + w) atomicAdd(&s_before[w], 1);
+            for (uint32_t left = s_map[b & 63]; left != 0; left &= left - 1) {
+                const int w = __builtin_ctz(left);
+                if (b != s_blk[w]) continue;
+                if (t < i0 + w || t >= i0 + w + s_len[w]) {
+                    atomicOr(&s_other, 1 << w);
+                    const int64_t before = t > 0 ? slot_mapping[t - 1] : -1;
+                    if (before < 0 || before >= capacity || static_cast<int>(before >> 4) != b) {
+                        atomicAdd(&s_segs[w], 1);
+                        if (t < i0 + w) atomicAdd(&s_before[w], 1);
+                    }
                 }
+                break;
             }
         }
     }
     __syncthreads();
-    const int others = s_other;
-    for (uint64_t left = mine; left != 0; left &= left - 1) {
+    // A block that other tokens land in too belongs to one of its segments, another one for other blocks: were it
+    // the first, the call's first windows would own nearly all blocks of tokens out of order.
+    uint64_t mine = starts, others = 0;
+    for (uint32_t left = s_other; left != 0; left &= left - 1) {
+        const int w = __builtin_ctz(left), b = s_blk[w];
+        const uint64_t same = __ballot(blk == b) & starts;
+        const int nth = __popcll(same & ((1ull << lane) - 1));  // of the block's starts here
+        mine &= ~same | __ballot(s_before[w] + nth == b % s_segs[w]);
+        others |= same;
+    }
+    int rank = 0;
+    for (uint64_t left = mine; left != 0; left &= left - 1, rank++) {
+        if (rank % static_cast<int>(gridDim.z) != static_cast<int>(blockIdx.z)) continue;
         const int l = __builtin_ctzll(left);
         const int i = i0 + l - 1;
-        if ((others >> (l - 1)) & 1) {
-            // One of the block's segments, another one for other blocks, has the workgroup that owns it: were it
-            // the first, the call's first windows would own nearly all blocks of tokens out of order.
-            if (s_before[l - 1] != s_blk[l - 1] % s_segs[l - 1]) continue;
+        if ((others >> l) & 1) {
             pa::append_int8_block<D, true>(k_new, v_new, IN_BF16, tok_stride, [&](int t) { return slot_mapping[t]; }, i, n_tok,
                                      k_cache, v_cache, k_scale, v_scale, k_absmax, v_absmax, num_kv_heads, capacity,
                                      static_cast<int32_t>(blockIdx.y), static_cast<int32_t>(gridDim.y));

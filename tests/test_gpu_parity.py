@@ -354,7 +354,7 @@ def test_append_int8_interleaved_bit_exact(stream, D, q_dtype, hkv, shift):
     interleaved token by token, a random order, a reversed one, rows written again and again in one segment of
     more than 64 tokens and in many; new K/V 16-byte aligned (shift 0) or one element off it."""
     rng = np.random.default_rng(290 + D + hkv)
-    nb = 40
+    nb = 140
     cfg = pa.make_config(num_q_heads=hkv, num_kv_heads=hkv, head_dim=D, kv_dtype=2, q_dtype=q_dtype,
                          num_blocks=nb)
     host = dict(kc=np.zeros((nb, hkv, 16, D), np.int8), vc=np.zeros((nb, hkv, 16, D), np.int8),
@@ -382,7 +382,7 @@ def test_append_int8_interleaved_bit_exact(stream, D, q_dtype, hkv, shift):
         pos = start + np.arange(n)
         return (blocks[:, pos // 16] * 16 + pos % 16).T
 
-    perm = rng.permutation(nb)
+    perm = rng.permutation(40)
     step(prompts(perm[:4].reshape(2, 2), 0, 9).reshape(-1))                       # 18 tokens
     step(prompts(perm[:4].reshape(2, 2), 9, 20).reshape(-1), (0.5, 4.0))
     step(prompts(perm[4:].reshape(6, 6), 3, 70).reshape(-1), (0.5, 2.0))           # 420 tokens, six at a time
@@ -391,6 +391,10 @@ def test_append_int8_interleaved_bit_exact(stream, D, q_dtype, hkv, shift):
     again = rng.integers(0, 16, 100) + 16 * perm[5]                                # one segment
     step(np.concatenate([again, [16 * perm[6] + 3], rng.integers(1, 16, 70) + 16 * perm[5], [-1], again[:3]]), (0.5, 3.0))
     step(rng.integers(0, 16, 300) + 16 * perm[rng.integers(7, 9, 300)], (0.5, 3.0))  # more segments than a list
+    # blocks alike in their low six bits: interleaved, in order, one token each
+    step(prompts(np.array([[3], [67], [131], [5], [69]]), 0, 7).reshape(-1), (0.5, 3.0))
+    step(np.concatenate([16 * b + np.arange(16) for b in (4, 68, 132)]), (0.5, 3.0))
+    step(16 * np.array([6, 70, 134, 7, 71, 135, 8, 72, 6, 136]) + np.arange(10), (0.5, 3.0))
 
 
 @pytest.mark.parametrize("old_scale,new_amax", [(0.5, 127.0), (0.0078125, 3.0), (0.2618793547153473, 95.5709228515625),
