@@ -1116,9 +1116,10 @@ __global__ __launch_bounds__(64 * decode_waves(D), D > 128 ? 1 : 2) void paged_d
 // over all context lengths, then block ids, then K/V, and a second launch that merges the ranges'
 // partials. Here the length, the row of the block table, Q and the new token are loaded together, so K/V
 // loads go out after one round trip, and no partial leaves the workgroup. Fused append steps, 32 / 8
-// heads of 128, bf16, us before -> now: 1 sequence of 333 tokens 12.6 -> 9.1 (calls
-// from Python, one after another); 16 of 333, 16.1 -> 11.7; 64 of 30 to 1000, 25.6 -> 24.9; 128 of 333, 38.7 -> 32.8. Eight waves measured slower throughout (64 of
-// 90: 14.5 against 8.9; at 172 registers a wave a CU holds one such workgroup).
+// heads of 128, bf16, us before -> now: 1 sequence of 333 tokens 12.6 -> 9.1 (calls from Python, one
+// after another); 16 of 333, 16.1 -> 11.7; 64 of 30 to 1000, 25.6 -> 24.9; 128 of 333, 38.7 -> 32.8. Eight
+// waves measured slower throughout (64 of 90: 14.5 against 8.9; at 172 registers a wave a CU holds one
+// such workgroup).
 //
 // A call of one sequence writes its new token here, once the workgroup has streamed the row. With more
 // sequences (a.append_after) a row may hold a block that another appends to, so the tokens wait for a launch
